@@ -93,21 +93,41 @@ enum
 
 enum
 {
-  MODE_STAGE = 0, /* RHS + LSRK update, clock advanced by the last block */
+  MODE_STAGE = 0, /* RHS + LSRK update */
   MODE_RHS = 1    /* write L(q, t) as FP64 into rhs, no update */
 };
 
+/* parameters of one stage of a subdomain: 64 bytes, one scalar load.
+ * parity: the stage reads q[parity] and writes q[parity ^ 1].
+ * dq_dead: the dq this stage writes is never read (the last stage of a step
+ *   of a scheme whose first stage has A = 0, every 2N-storage scheme here).
+ *   Where dq is rebuilt from the states (rec), no stage stores it.
+ * rec: B[s-1] times the old dq is q[parity] - q[parity ^ 1], and a holds
+ *   A[s] / B[s-1].
+ * g, sw, cw: ricker(t_stage), and sin, cos(omega t_stage) of the
+ *   manufactured forcing. */
+struct StageSlot
+{
+  int parity, dq_dead, rec, pad;
+  double a, b, dt, g, sw, cw;
+};
+
 /* device-resident clock of one subdomain; all dynamic state lives here so a
- * captured graph can be replayed */
+ * captured graph can be replayed.  `ctx` holds the parameters of the next
+ * CLOCK_SLOTS stages, counted from `stage`; a launch names its slot, so a
+ * run of up to CLOCK_SLOTS stages (eight steps of five stages) needs one
+ * clock kernel after its last stage.  With a one-thread clock kernel after
+ * every stage, that kernel took 2.6 us of the 8.3 us of a small stage
+ * (16 x 16 acoustic, FP64) and 4.6 us beside stages of 55-400 us: a chain of
+ * dependent reads and FP64 exp and sincos. */
+constexpr int CLOCK_SLOTS = 40;
 struct Clock
 {
-  double t;            /* time at the start of the current step */
-  double dt;           /* step size */
-  long long stage;     /* stages completed since set_fields */
-  unsigned int arrive; /* blocks of the current launch that finished */
-  unsigned int pad;
-  double g;            /* ricker(t_stage) of the stage about to run */
-  double sw, cw;       /* sin, cos(omega t_stage) for the manufactured forcing */
+  double t;        /* time at the start of the current step */
+  double dt;       /* step size */
+  long long stage; /* stages completed since set_fields */
+  long long pad[5];
+  StageSlot ctx[CLOCK_SLOTS];
 };
 
 /* everything a stage needs about one subdomain (passed by value or read
@@ -210,6 +230,7 @@ struct GlueArgs
   const SubDev *subs; /* the batch's descriptors */
   const MortarGroup *groups;
   int ngroups;
+  int slot; /* as LaunchArgs::slot */
   const void *ops; /* glue_ops8_index table, arithmetic type */
   void *buf;       /* face fluctuation blocks */
 };
@@ -277,10 +298,11 @@ struct LaunchArgs
   /* node-parallel stage: one block per task even where the one-element
    * kernel takes one element per block (an order launched beside others) */
   int whole_tasks;
-  double t_rhs;  /* time for MODE_RHS */
-  double g_rhs;  /* ricker(t_rhs) */
-  double sw_rhs; /* sin(omega t_rhs) */
-  double cw_rhs; /* cos(omega t_rhs) */
+  /* stages launched since the clocks were last advanced: the stage's entry
+   * of Clock::ctx */
+  int slot;
+  /* MODE_RHS: ricker(t), sin and cos(omega t) at the caller's time */
+  double g_rhs, sw_rhs, cw_rhs;
 };
 
 /* element-major offset of (element, field, node) */
@@ -342,50 +364,12 @@ __device__ __forceinline__ double ricker(double f0, double t0, double t)
   return (1 - 2 * a) * exp(-a);
 }
 
-/* time-dependent source/forcing scalars of the stage that starts next.  Kept
- * out of line: only the clock-advancing thread runs it, and inlining the FP64
- * exp/sincos would raise the register budget of the whole stage kernel. */
-__device__ __noinline__ void clock_scalars(const SubDev &sd, Clock *c)
-{
-  const long long st = c->stage;
-  const double ts = c->t + sd.C[(int)(st % sd.nstages)] * c->dt;
-  if (sd.src_elem >= 0)
-    c->g = ricker(sd.src_f0, sd.src_t0, ts);
-  if (sd.mms)
-  {
-    double sv, cv;
-    sincos(sd.mms_omega * ts, &sv, &cv);
-    c->sw = sv;
-    c->cw = cv;
-  }
-}
-
-/* advance a subdomain's clock by one stage (run by one thread, in a kernel
- * launched after the stage kernel, so no block of the stage reads the clock
- * while it changes) */
-__device__ __forceinline__ void clock_advance(const SubDev &sd)
-{
-  gptr<Clock> c = glob(sd.clock);
-  const long long st = c->stage + 1;
-  c->stage = st;
-  if (st % sd.nstages == 0)
-    c->t = c->t + c->dt;
-  clock_scalars(sd, (Clock *)c);
-}
-
-/* stage parameters of the subdomain read at the start of a task */
+/* stage parameters of a task's subdomain */
 struct StageCtx
 {
-  int parity;
-  /* the dq this stage writes is never read: the last stage of a step of a
-   * scheme whose first stage has A = 0 (every 2N-storage scheme here).
-   * Where dq is rebuilt from the states (rec), no stage stores it */
-  int dq_dead;
-  double a, b, dt, t;
-  double g, sw, cw;
-  /* B[s-1] times the old dq is q[parity] - q[parity ^ 1], and a holds
-   * A[s] / B[s-1] */
-  int rec;
+  int parity, dq_dead, rec;
+  double a, b, dt;
+  cptr<StageSlot> slot;
 };
 
 /* SD: SubDev, possibly qualified with the constant address space.  The
@@ -395,38 +379,31 @@ template <class SD>
 __device__ __forceinline__ StageCtx stage_ctx(const SD &sd, const LaunchArgs &a)
 {
   StageCtx c;
-  const int mode = a.mode;
-  const double t_rhs = a.t_rhs;
-  cptr<Clock> clk = cglob((const Clock *)sd.clock);
-  if (mode == MODE_RHS)
-  {
-    c.parity = (int)(clk->stage & 1);
-    c.dq_dead = 0;
-    c.rec = 0;
-    c.a = 0;
-    c.b = 0;
-    c.dt = 0;
-    c.t = t_rhs;
-    c.g = a.g_rhs;
-    c.sw = a.sw_rhs;
-    c.cw = a.cw_rhs;
-    return c;
-  }
-  c.g = clk->g;
-  c.sw = clk->sw;
-  c.cw = clk->cw;
-  const long long st = clk->stage;
-  const int s = (int)(st % sd.nstages);
-  c.parity = (int)(st & 1);
-  c.rec = sd.dq_rec;
-  c.dq_dead = s == sd.nstages - 1 && sd.A[0] == 0.0;
-  c.a = sd.AB[s];
-  c.b = sd.B[s];
-  c.dt = clk->dt;
-  c.t = clk->t + sd.C[s] * c.dt;
+  c.slot = cglob((const StageSlot *)((const Clock *)sd.clock)->ctx) + a.slot;
+  const bool stage = a.mode != MODE_RHS;
+  c.parity = c.slot->parity;
+  c.dq_dead = stage ? c.slot->dq_dead : 0;
+  c.rec = stage ? c.slot->rec : 0;
+  c.a = stage ? c.slot->a : 0.0;
+  c.b = stage ? c.slot->b : 0.0;
+  c.dt = stage ? c.slot->dt : 0.0;
   return c;
 }
 
+/* the source and forcing scalars, loaded only where a task needs them: held
+ * from the start of a task they cost the stage kernels registers */
+__device__ __forceinline__ double stage_g(const StageCtx &c, const LaunchArgs &a)
+{
+  return a.mode == MODE_RHS ? a.g_rhs : c.slot->g;
+}
+__device__ __forceinline__ double stage_sw(const StageCtx &c, const LaunchArgs &a)
+{
+  return a.mode == MODE_RHS ? a.sw_rhs : c.slot->sw;
+}
+__device__ __forceinline__ double stage_cw(const StageCtx &c, const LaunchArgs &a)
+{
+  return a.mode == MODE_RHS ? a.cw_rhs : c.slot->cw;
+}
 
 /* the neighbour's node facing node nm of face f (non-glued faces): the
  * upload admits only axis-aligned connectivity, a neighbour meeting face f

@@ -39,7 +39,8 @@ constexpr int GS = 72;
 /* face trace (v, sigma[.][A]) of one element face into LDS, lane = padded
  * node */
 template <class TS, class TC, class SD>
-__device__ __forceinline__ void load_trace(const SD &sd, int32_t e, int f, TC *tr, int lane)
+__device__ __forceinline__ void load_trace(const SD &sd, int slot, int32_t e, int f, TC *tr,
+                                           int lane)
 {
   const int n1 = sd.N + 1, np = n1 * n1 * n1, A = f >> 1;
   const int a = lane % GP, b = lane / GP;
@@ -50,7 +51,7 @@ __device__ __forceinline__ void load_trace(const SD &sd, int32_t e, int f, TC *t
       tr[c * GS + lane] = TC(0);
     return;
   }
-  const int parity = (int)(cglob((const Clock *)sd.clock)->stage & 1);
+  const int parity = cglob((const Clock *)sd.clock)->ctx[slot].parity;
   gptr<const TS> q = glob(static_cast<const TS *>(sd.q[parity])) + (size_t)e * 9 * np +
                      face_node<3>(f, n1, a, b);
 #pragma unroll
@@ -157,7 +158,7 @@ __global__ __launch_bounds__(64 * GLUE_WAVES) void mortar_kernel(GlueArgs a)
 
   /* ---- every load of the group ---- */
   if (m == 0)
-    load_trace<TS, TC>(B, b_elem, b_face, tb, lane);
+    load_trace<TS, TC>(B, a.slot, b_elem, b_face, tb, lane);
   /* the mortar's orders and its six operators (glue_ops8_index blocks):
    * interpolation of the s face (Is) and of the b face along each axis
    * (Ia, Ib) to the mortar grid, and the mass projections back (Ws; Wa,
@@ -169,7 +170,7 @@ __global__ __launch_bounds__(64 * GLUE_WAVES) void mortar_kernel(GlueArgs a)
   if (mine)
   {
     const auto &S = *(cglob(a.subs) + gp->s_sub[m]);
-    load_trace<TS, TC>(S, gp->s_elem[m], gp->s_face[m], ts[m], lane);
+    load_trace<TS, TC>(S, a.slot, gp->s_elem[m], gp->s_face[m], ts[m], lane);
     Ns = S.N;
     const int Ng = gp->s_ng[m] > 0 ? gp->s_ng[m] : (Ns > Nb ? Ns : Nb);
     const int quad = nm == 1 ? quad0 : m;

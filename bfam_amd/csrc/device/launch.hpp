@@ -64,10 +64,11 @@ hipError_t launch_elastic_plain(int N, const LaunchArgs &a, int grid,
                                 hipStream_t s);
 hipError_t launch_acoustic_plain(int N, const LaunchArgs &a, int grid,
                                  hipStream_t s);
-hipError_t launch_plain_update(const SubDev *sd_dev, size_t ndof,
+hipError_t launch_plain_update(const SubDev *sd_dev, int slot, size_t ndof,
                                hipStream_t s, int nblocks);
-/* advance the clocks of nsubs device descriptors by one stage */
-hipError_t launch_clock_advance(const SubDev *subs, int nsubs, hipStream_t s);
+/* advance the clocks of nsubs device descriptors by m stages and refill the
+ * stage parameters from slot `first` on */
+hipError_t launch_clock_advance(const SubDev *subs, int nsubs, int m, int first, hipStream_t s);
 hipError_t launch_mortar(int prec, const GlueArgs &a, hipStream_t s);
 
 /* field transfer between adapted meshes: one source or destination

@@ -13,14 +13,12 @@ namespace bfamx
 {
 
 /* dq = A dq + dt rhs;  q = q + B dq  over all DOF */
-__global__ __launch_bounds__(256) void plain_update_kernel(const SubDev *sdp,
+__global__ __launch_bounds__(256) void plain_update_kernel(const SubDev *sdp, int slot,
                                                           size_t ndof)
 {
   const SubDev &sd = *(const SubDev *)glob(sdp);
-  gptr<const Clock> clk = glob((const Clock *)sd.clock);
-  const long long st = clk->stage;
-  const int s = (int)(st % sd.nstages);
-  const double a = sd.A[s], b = sd.B[s], dt = clk->dt;
+  cptr<StageSlot> cx = cglob((const StageSlot *)sd.clock->ctx) + slot;
+  const double a = cx->a, b = cx->b, dt = cx->dt;
   gptr<double> q = glob(static_cast<double *>(sd.q[0]));
   gptr<double> dq = glob(static_cast<double *>(sd.dq));
   gptr<const double> rhs = glob((const double *)sd.rhs);
@@ -33,26 +31,73 @@ __global__ __launch_bounds__(256) void plain_update_kernel(const SubDev *sdp,
   }
 }
 
-/* one thread per subdomain: advance its clock past the stage just run */
-__global__ void clock_advance_kernel(const SubDev *subs, int nsubs)
+/* One wavefront per subdomain: advance its clock past the m stages just run
+ * and write the parameters of the next CLOCK_SLOTS stages, lane i those of
+ * the i-th, from slot `first` on.  It runs after the stage kernels, so no
+ * block of a stage reads the clock while it changes.  Time advances by one
+ * addition of dt per step, in each lane, so that it has the same bits
+ * however the stages were divided into runs. */
+__global__ __launch_bounds__(64) void clock_advance_kernel(const SubDev *subs, int m, int first)
 {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < nsubs)
-    clock_advance(*(const SubDev *)(glob(subs) + i));
+  const SubDev &sd = *(const SubDev *)(glob(subs) + blockIdx.x);
+  gptr<Clock> c = glob(sd.clock);
+  const int i = threadIdx.x, S = sd.nstages;
+  const long long st0 = c->stage;
+  const double dt = c->dt;
+  double t = c->t;
+  int s = (int)(st0 % S); /* stage within the step */
+  for (int k = 0; k < m; ++k)
+    if (++s == S)
+    {
+      s = 0;
+      t = t + dt;
+    }
+  const int s0 = s;
+  const double t0 = t;
+  __syncthreads(); /* every lane has read the clock */
+  if (i == 0)
+  {
+    c->stage = st0 + m;
+    c->t = t0;
+  }
+  if (i < first || i >= CLOCK_SLOTS)
+    return;
+  for (int k = 0; k < i; ++k)
+    if (++s == S)
+    {
+      s = 0;
+      t = t + dt;
+    }
+  gptr<StageSlot> x = glob((StageSlot *)sd.clock->ctx) + i;
+  x->parity = (int)((st0 + m + i) & 1);
+  x->dq_dead = s == S - 1 && sd.A[0] == 0.0;
+  x->rec = sd.dq_rec;
+  x->a = sd.AB[s];
+  x->b = sd.B[s];
+  x->dt = dt;
+  const double ts = t + sd.C[s] * dt;
+  if (sd.src_elem >= 0)
+    x->g = ricker(sd.src_f0, sd.src_t0, ts);
+  if (sd.mms)
+  {
+    double sv, cv;
+    sincos(sd.mms_omega * ts, &sv, &cv);
+    x->sw = sv;
+    x->cw = cv;
+  }
 }
 
-hipError_t launch_clock_advance(const SubDev *subs, int nsubs, hipStream_t s)
+hipError_t launch_clock_advance(const SubDev *subs, int nsubs, int m, int first, hipStream_t s)
 {
-  hipLaunchKernelGGL(clock_advance_kernel, dim3((nsubs + 63) / 64), dim3(64), 0,
-                     s, subs, nsubs);
+  hipLaunchKernelGGL(clock_advance_kernel, dim3(nsubs), dim3(64), 0, s, subs, m, first);
   return hipGetLastError();
 }
 
-hipError_t launch_plain_update(const SubDev *sd_dev, size_t ndof,
+hipError_t launch_plain_update(const SubDev *sd_dev, int slot, size_t ndof,
                                hipStream_t s, int nblocks)
 {
   hipLaunchKernelGGL(plain_update_kernel, dim3(nblocks), dim3(256), 0, s,
-                     sd_dev, ndof);
+                     sd_dev, slot, ndof);
   return hipGetLastError();
 }
 

@@ -13,10 +13,12 @@
 #include <hip/hip_runtime.h>
 
 #include <math.h>
+#include <stddef.h>
 #include <stdlib.h>
 #include <string.h>
 
 #include <algorithm>
+#include <atomic>
 #include <vector>
 
 #include "../bfamx_internal.h"
@@ -99,6 +101,9 @@ struct bfamx_subdomain
    * stages launched since (glued batch members must agree on all three) */
   double t0_set, dt_set;
   long long stages_run;
+  /* whose descriptor's source and forcing the clock's slots were computed
+   * with: the subdomain's own (0), or the copy of the batch of that id */
+  unsigned long long clock_by;
   bfamx_lsrk_t lsrk;
   bfamx_glue_t *glue; /* set while faces of this subdomain are glued */
 };
@@ -127,6 +132,7 @@ struct bfamx_glue
 struct bfamx_batch
 {
   bfamx_device_t *dev;
+  unsigned long long id; /* of no other batch of the process; not 0 */
   std::vector<bfamx_subdomain_t *> subs;
   SubDev *d_subs;
   Task *d_tasks;
@@ -458,6 +464,48 @@ static int push_sub(bfamx_subdomain_t *s)
   return BFAMX_OK;
 }
 
+/* the scalar members of Clock, as the host reads and sets them */
+struct ClockHead
+{
+  double t, dt;
+  long long stage;
+};
+static_assert(offsetof(Clock, stage) == offsetof(ClockHead, stage), "head of Clock");
+
+static int read_clock(bfamx_subdomain_t *s, ClockHead *c)
+{
+  HIPCHK(hipStreamSynchronize(s->dev->stream));
+  HIPCHK(hipMemcpy(c, s->d_clock, sizeof(*c), hipMemcpyDeviceToHost));
+  return BFAMX_OK;
+}
+
+/* recompute the parameters of the stages about to run, after the clock or
+ * the subdomain's descriptor changed */
+static int refresh_clock(bfamx_subdomain_t *s)
+{
+  s->clock_by = 0;
+  HIPCHK(launch_clock_advance(s->d_sub, 1, 0, 0, s->dev->stream));
+  return BFAMX_OK;
+}
+
+/* before a run of stages from the n descriptors d_subs of the members (`by`:
+ * as clock_by): slots that another descriptor computed are recomputed with
+ * these, except the stage about to run, whose parameters the clock's last
+ * advance fixed */
+static int own_clocks(bfamx_device_t *d, bfamx_subdomain_t *const *subs, int n,
+                      const SubDev *d_subs, unsigned long long by)
+{
+  bool all = true;
+  for (int i = 0; i < n; ++i)
+  {
+    all = all && subs[i]->clock_by == by;
+    subs[i]->clock_by = by;
+  }
+  if (!all)
+    HIPCHK(launch_clock_advance(d_subs, n, 0, 1, d->stream));
+  return BFAMX_OK;
+}
+
 extern "C" int bfamx_subdomain_upload(bfamx_device_t *dev,
                                       const bfamx_dgx_t *sub,
                                       const bfamx_physics_desc_t *phys,
@@ -740,6 +788,8 @@ extern "C" int bfamx_subdomain_upload(bfamx_device_t *dev,
     }
   }
   rc = push_sub(s);
+  if (!rc)
+    rc = refresh_clock(s);
   if (rc)
     goto fail;
   *out = s;
@@ -781,24 +831,6 @@ static double host_ricker(double f0, double t0, double t)
   return (1 - 2 * a) * exp(-a);
 }
 
-/* recompute the time scalars of the stage about to run (host side) */
-static int refresh_clock(bfamx_subdomain_t *s)
-{
-  Clock c;
-  HIPCHK(hipStreamSynchronize(s->dev->stream));
-  HIPCHK(hipMemcpy(&c, s->d_clock, sizeof(c), hipMemcpyDeviceToHost));
-  const double ts = c.t + s->h.C[(int)(c.stage % s->h.nstages)] * c.dt;
-  if (s->h.src_elem >= 0)
-    c.g = host_ricker(s->h.src_f0, s->h.src_t0, ts);
-  if (s->h.mms)
-  {
-    c.sw = sin(s->h.mms_omega * ts);
-    c.cw = cos(s->h.mms_omega * ts);
-  }
-  HIPCHK(hipMemcpy(s->d_clock, &c, sizeof(c), hipMemcpyHostToDevice));
-  return BFAMX_OK;
-}
-
 extern "C" int bfamx_set_source(bfamx_subdomain_t *s, int32_t elem,
                                 const double *weights, const double *amp,
                                 double f0, double t0)
@@ -806,6 +838,8 @@ extern "C" int bfamx_set_source(bfamx_subdomain_t *s, int32_t elem,
   if (!s || !weights || !amp || elem < 0 || elem >= s->K)
     return bfamx_fail(BFAMX_EINVAL, "bfamx_set_source: bad arguments");
   int rc;
+  /* stages in flight keep the source they were launched with */
+  HIPCHK(hipStreamSynchronize(s->dev->stream));
   if (!s->h.src_wt)
   {
     void *p;
@@ -838,6 +872,7 @@ extern "C" int bfamx_set_forcing_mms(bfamx_subdomain_t *s, double k,
   if (!s || !F || s->physics != BFAMX_ELASTIC3D)
     return bfamx_fail(BFAMX_EINVAL, "bfamx_set_forcing_mms: elastic only");
   const int n1 = s->N + 1;
+  HIPCHK(hipStreamSynchronize(s->dev->stream));
   if (!s->h.mms_tab)
   {
     /* sin/cos(k x) at the element's node coordinates, per axis (static in
@@ -914,10 +949,7 @@ extern "C" int bfamx_set_fields(bfamx_subdomain_t *s,
   }
   if (s->h.dq)
     HIPCHK(hipMemset(s->h.dq, 0, (s->rate_fp32 ? 4 : 8) * ndof));
-  Clock c;
-  memset(&c, 0, sizeof(c));
-  c.t = t0;
-  c.dt = dt;
+  const ClockHead c = {t0, dt, 0};
   HIPCHK(hipMemcpy(s->d_clock, &c, sizeof(c), hipMemcpyHostToDevice));
   s->fields_set = 1;
   s->t0_set = t0;
@@ -928,9 +960,10 @@ extern "C" int bfamx_set_fields(bfamx_subdomain_t *s,
 
 static int current_parity(bfamx_subdomain_t *s, int *parity)
 {
-  Clock c;
-  HIPCHK(hipStreamSynchronize(s->dev->stream));
-  HIPCHK(hipMemcpy(&c, s->d_clock, sizeof(c), hipMemcpyDeviceToHost));
+  ClockHead c;
+  int rc = read_clock(s, &c);
+  if (rc)
+    return rc;
   *parity = s->prec == BFAMX_FP64_PLAIN ? 0 : (int)(c.stage & 1);
   return BFAMX_OK;
 }
@@ -939,9 +972,10 @@ extern "C" int bfamx_get_time(bfamx_subdomain_t *s, double *t, int64_t *stages)
 {
   if (!s)
     return bfamx_fail(BFAMX_EINVAL, "NULL subdomain");
-  Clock c;
-  HIPCHK(hipStreamSynchronize(s->dev->stream));
-  HIPCHK(hipMemcpy(&c, s->d_clock, sizeof(c), hipMemcpyDeviceToHost));
+  ClockHead c;
+  int rc = read_clock(s, &c);
+  if (rc)
+    return rc;
   if (t)
     *t = c.t;
   if (stages)
@@ -1134,8 +1168,6 @@ static int run_fused(bfamx_subdomain_t *s, const LaunchArgs &a)
   else
     e = launch_elastic_line(s->prec, s->N, a, grid_line(s->dev, s->prec, s->N, a.ntasks),
                             s->dev->stream, kernel_dyn(s->dev, s->prec, s->N, 0));
-  if (e == hipSuccess && a.mode == MODE_STAGE)
-    e = launch_clock_advance(s->d_sub, 1, s->dev->stream);
   if (e != hipSuccess)
     return bfamx_fail(BFAMX_EHIP, "stage launch failed: %s", hipGetErrorString(e));
   return BFAMX_OK;
@@ -1152,25 +1184,46 @@ static int run_plain_rhs(bfamx_subdomain_t *s, const LaunchArgs &a)
   return BFAMX_OK;
 }
 
-static int stage_once(bfamx_subdomain_t *s)
+/* the kernels of the stage whose parameters are in `slot` of the clock */
+static int stage_once(bfamx_subdomain_t *s, int slot)
 {
+  LaunchArgs a = launch_args(s, MODE_STAGE);
+  a.slot = slot;
   if (s->prec == BFAMX_FP64_PLAIN)
   {
-    int rc = run_plain_rhs(s, launch_args(s, MODE_STAGE));
+    int rc = run_plain_rhs(s, a);
     if (rc)
       return rc;
     const size_t ndof = (size_t)s->K * s->nf * s->Np;
     const int nb = (int)((ndof + 255) / 256 < (size_t)s->dev->num_cu * 16
                              ? (ndof + 255) / 256
                              : (size_t)s->dev->num_cu * 16);
-    hipError_t e = launch_plain_update(s->d_sub, ndof, s->dev->stream, nb);
-    if (e == hipSuccess)
-      e = launch_clock_advance(s->d_sub, 1, s->dev->stream);
+    hipError_t e = launch_plain_update(s->d_sub, slot, ndof, s->dev->stream, nb);
     if (e != hipSuccess)
       return bfamx_fail(BFAMX_EHIP, "update launch failed: %s", hipGetErrorString(e));
     return BFAMX_OK;
   }
-  return run_fused(s, launch_args(s, MODE_STAGE));
+  return run_fused(s, a);
+}
+
+/* n stages, the clock advanced once per CLOCK_SLOTS of them; where a launch
+ * fails, the clock still counts the stages launched before it */
+static int run_stages(bfamx_subdomain_t *s, long long n)
+{
+  int rc = own_clocks(s->dev, &s, 1, s->d_sub, 0);
+  while (n > 0 && !rc)
+  {
+    const int m = n < CLOCK_SLOTS ? (int)n : CLOCK_SLOTS;
+    int k = 0;
+    while (k < m && !(rc = stage_once(s, k)))
+      ++k;
+    const hipError_t e = launch_clock_advance(s->d_sub, 1, k, 0, s->dev->stream);
+    if (e != hipSuccess && !rc)
+      rc = bfamx_fail(BFAMX_EHIP, "clock launch failed: %s", hipGetErrorString(e));
+    s->stages_run += k;
+    n -= m;
+  }
+  return rc;
 }
 
 extern "C" int bfamx_stage(bfamx_subdomain_t *s)
@@ -1181,10 +1234,7 @@ extern "C" int bfamx_stage(bfamx_subdomain_t *s)
     return bfamx_fail(BFAMX_ESTATE, "bfamx_stage: no state set");
   if (s->glue)
     return bfamx_fail(BFAMX_ESTATE, "glued subdomains advance through their batch");
-  int rc = stage_once(s);
-  if (!rc)
-    ++s->stages_run;
-  return rc;
+  return run_stages(s, 1);
 }
 
 extern "C" int bfamx_step(bfamx_subdomain_t *s, int nsteps)
@@ -1195,15 +1245,7 @@ extern "C" int bfamx_step(bfamx_subdomain_t *s, int nsteps)
     return bfamx_fail(BFAMX_ESTATE, "bfamx_step: no state set");
   if (s->glue)
     return bfamx_fail(BFAMX_ESTATE, "glued subdomains advance through their batch");
-  for (int i = 0; i < nsteps; ++i)
-    for (int st = 0; st < s->h.nstages; ++st)
-    {
-      int rc = stage_once(s);
-      if (rc)
-        return rc;
-      ++s->stages_run;
-    }
-  return BFAMX_OK;
+  return run_stages(s, (long long)nsteps * s->h.nstages);
 }
 
 static int rhs_one(bfamx_subdomain_t *s, double t, double *const *rhs);
@@ -1224,7 +1266,6 @@ extern "C" int bfamx_rhs(bfamx_subdomain_t *s, double t, double *const *rhs)
 static int rhs_launch(bfamx_subdomain_t *s, double t)
 {
   LaunchArgs a = launch_args(s, MODE_RHS);
-  a.t_rhs = t;
   a.g_rhs = s->h.src_elem >= 0 ? host_ricker(s->h.src_f0, s->h.src_t0, t) : 0.0;
   a.sw_rhs = s->h.mms ? sin(s->h.mms_omega * t) : 0.0;
   a.cw_rhs = s->h.mms ? cos(s->h.mms_omega * t) : 0.0;
@@ -1383,9 +1424,10 @@ static int mms_partials(bfamx_subdomain_t *s, const double *A, double *out4)
 {
   if (!s || !A || !s->h.mms_tab)
     return bfamx_fail(BFAMX_EINVAL, "MMS error: no forcing set");
-  Clock c;
-  HIPCHK(hipStreamSynchronize(s->dev->stream));
-  HIPCHK(hipMemcpy(&c, s->d_clock, sizeof(c), hipMemcpyDeviceToHost));
+  ClockHead c;
+  int rc = read_clock(s, &c);
+  if (rc)
+    return rc;
   const int parity = s->prec == BFAMX_FP64_PLAIN ? 0 : (int)(c.stage & 1);
   /* the state is at a step boundary only when stage % nstages == 0 */
   hipError_t e = launch_mms_error(s->h, s->state_fp32, parity, A,
@@ -1462,8 +1504,10 @@ extern "C" int bfamx_batch_create(bfamx_device_t *dev,
   }
   if (N < 0 && physics != BFAMX_ELASTIC3D)
     return bfamx_fail(BFAMX_EUNSUPPORTED, "mixed orders: elastic only");
+  static std::atomic<unsigned long long> next_id{1};
   bfamx_batch_t *b = new bfamx_batch_t();
   b->dev = dev;
+  b->id = next_id++;
   b->subs.assign(subs, subs + nsubs);
   b->physics = physics;
   b->prec = prec;
@@ -1616,6 +1660,7 @@ static GlueArgs glue_args(const bfamx_batch_t *b)
   g.ngroups = b->glue->ngroups;
   g.ops = b->glue->d_ops;
   g.buf = b->glue->d_buf;
+  g.slot = 0;
   return g;
 }
 
@@ -1706,7 +1751,8 @@ static hipError_t launch_batch_kernels(bfamx_batch_t *b, const LaunchArgs &a,
   return e;
 }
 
-static int batch_stage(bfamx_batch_t *b)
+/* the kernels of the stage whose parameters are in `slot` of the clocks */
+static int batch_stage(bfamx_batch_t *b, int slot)
 {
   LaunchArgs a;
   memset(&a, 0, sizeof(a));
@@ -1716,17 +1762,42 @@ static int batch_stage(bfamx_batch_t *b)
   a.mode = MODE_STAGE;
   a.xcd_remap = b->dev->xcd_remap;
   a.nxcd = b->dev->num_xcd;
+  a.slot = slot;
   const int grid = grid_for(b->dev, b->ntasks);
   hipError_t e = hipSuccess;
   if (b->glue)
-    e = launch_mortar(b->prec, glue_args(b), b->dev->stream);
+  {
+    GlueArgs g = glue_args(b);
+    g.slot = slot;
+    e = launch_mortar(b->prec, g, b->dev->stream);
+  }
   if (e == hipSuccess)
     e = launch_batch_kernels(b, a, grid);
-  if (e == hipSuccess)
-    e = launch_clock_advance(b->d_subs, (int)b->subs.size(), b->dev->stream);
   if (e != hipSuccess)
     return bfamx_fail(BFAMX_EHIP, "batch stage launch: %s", hipGetErrorString(e));
   return BFAMX_OK;
+}
+
+/* n stages, the clocks advanced once per CLOCK_SLOTS of them (also where a
+ * launch fails, by the stages launched before it); *done: stages launched */
+static int batch_run(bfamx_batch_t *b, long long n, long long *done)
+{
+  int rc = BFAMX_OK;
+  *done = 0;
+  while (n > 0 && !rc)
+  {
+    const int m = n < CLOCK_SLOTS ? (int)n : CLOCK_SLOTS;
+    int k = 0;
+    while (k < m && !(rc = batch_stage(b, k)))
+      ++k;
+    const hipError_t e =
+        launch_clock_advance(b->d_subs, (int)b->subs.size(), k, 0, b->dev->stream);
+    if (e != hipSuccess && !rc)
+      rc = bfamx_fail(BFAMX_EHIP, "clock launch failed: %s", hipGetErrorString(e));
+    *done += k;
+    n -= m;
+  }
+  return rc;
 }
 
 /* stages of one step: bfamx_batch_create admits one stage count only */
@@ -1767,16 +1838,16 @@ extern "C" int bfamx_batch_step(bfamx_batch_t *b, int nsteps)
   int rc = batch_ready(b);
   if (rc)
     return rc;
-  const int ns = batch_nstages(b);
-  for (int i = 0; i < nsteps * ns; ++i)
-  {
-    rc = batch_stage(b);
-    if (rc)
-      return rc;
-    for (auto *s : b->subs)
-      ++s->stages_run;
-  }
-  return BFAMX_OK;
+  if (nsteps == 0)
+    return BFAMX_OK;
+  rc = own_clocks(b->dev, b->subs.data(), (int)b->subs.size(), b->d_subs, b->id);
+  if (rc)
+    return rc;
+  long long done;
+  rc = batch_run(b, (long long)nsteps * batch_nstages(b), &done);
+  for (auto *s : b->subs)
+    s->stages_run += done;
+  return rc;
 }
 
 extern "C" int bfamx_batch_capture(bfamx_batch_t *b, int nsteps)
@@ -1796,10 +1867,8 @@ extern "C" int bfamx_batch_capture(bfamx_batch_t *b, int nsteps)
   hipStream_t st = b->dev->stream;
   HIPCHK(hipStreamSynchronize(st));
   HIPCHK(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
-  const int ns = batch_nstages(b);
-  int rc = BFAMX_OK;
-  for (int i = 0; i < nsteps * ns && rc == BFAMX_OK; ++i)
-    rc = batch_stage(b);
+  long long done;
+  const int rc = batch_run(b, (long long)nsteps * batch_nstages(b), &done);
   hipGraph_t g = NULL;
   hipError_t e = hipStreamEndCapture(st, &g);
   if (rc)
@@ -1821,6 +1890,9 @@ extern "C" int bfamx_batch_launch_graph(bfamx_batch_t *b)
   if (!b || !b->exec)
     return bfamx_fail(BFAMX_ESTATE, "bfamx_batch_launch_graph: not captured");
   int rc = batch_ready(b);
+  if (rc)
+    return rc;
+  rc = own_clocks(b->dev, b->subs.data(), (int)b->subs.size(), b->d_subs, b->id);
   if (rc)
     return rc;
   HIPCHK(hipGraphLaunch(b->exec, b->dev->stream));
@@ -2643,10 +2715,7 @@ extern "C" int bfamx_transfer_fields(const bfamx_transfer_maps_t *m,
     const size_t ndof = (size_t)s->K * s->nf * s->Np;
     if (s->h.dq)
       HIPCHK(hipMemset(s->h.dq, 0, (s->rate_fp32 ? 4 : 8) * ndof));
-    Clock c;
-    memset(&c, 0, sizeof(c));
-    c.t = t;
-    c.dt = dt;
+    const ClockHead c = {t, dt, 0};
     HIPCHK(hipMemcpy(s->d_clock, &c, sizeof(c), hipMemcpyHostToDevice));
     s->fields_set = 1;
     s->t0_set = t;

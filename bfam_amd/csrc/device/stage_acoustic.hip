@@ -24,7 +24,7 @@ template <int N, int EPB, class T> struct AcousticSmem
 
 template <int N, int EPB, class P, int PART = PART_FUSED, class SD>
 __device__ __forceinline__ void acoustic_task(const SD &sd, const Task &tk,
-                                              const StageCtx &cx, int mode,
+                                              const StageCtx &cx, const LaunchArgs &la,
                                               char *smem)
 {
   using TS = typename P::TS;
@@ -173,14 +173,14 @@ __device__ __forceinline__ void acoustic_task(const SD &sd, const Task &tk,
 
   if (PART != PART_SURFACE && e == sd.src_elem)
   {
-    const TC g = (TC)cx.g;
+    const TC g = (TC)stage_g(cx, la);
     const TC w = src_tab<TC>(sd)[n];
 #pragma unroll
     for (int f = 0; f < NF; ++f)
       rate[f] += w * (TC)sd.src_amp[f] * g;
   }
 
-  if (mode == MODE_RHS || PART != PART_FUSED)
+  if (la.mode == MODE_RHS || PART != PART_FUSED)
   {
 #pragma unroll
     for (int f = 0; f < NF; ++f)
@@ -228,7 +228,7 @@ acoustic_stage_kernel(LaunchArgs a)
     const Task tk = load_task(a.tasks, ti);
     const auto &sd = *(cglob(a.subs) + tk.sub);
     const StageCtx cx = stage_ctx(sd, a);
-    acoustic_task<N, EPB, P>(sd, tk, cx, a.mode, smem);
+    acoustic_task<N, EPB, P>(sd, tk, cx, a, smem);
     __syncthreads();
   }
 }
@@ -282,7 +282,7 @@ acoustic_part_kernel(LaunchArgs a)
     const Task tk = load_task(a.tasks, ti);
     const auto &sd = *(cglob(a.subs) + tk.sub);
     const StageCtx cx = stage_ctx(sd, a);
-    acoustic_task<N, EPB, P64, PART>(sd, tk, cx, a.mode, smem);
+    acoustic_task<N, EPB, P64, PART>(sd, tk, cx, a, smem);
     __syncthreads();
   }
 }

@@ -112,7 +112,7 @@ __device__ __forceinline__ void block_to_lds(gptr<const float> src, float *dst,
 
 template <int N, int EPB, class P, int PART = PART_FUSED, class SD>
 __device__ __forceinline__ void elastic_task(const SD &sd, const Task &tk,
-                                             const StageCtx &cx, int mode,
+                                             const StageCtx &cx, const LaunchArgs &la,
                                              char *smem)
 {
   using TS = typename P::TS;
@@ -197,7 +197,7 @@ __device__ __forceinline__ void elastic_task(const SD &sd, const Task &tk,
    * non-temporally: L2 then keeps the states that neighbouring blocks
    * gather their face traces from (FP32 48^3 N=7: 1.635 -> 1.548 ms per
    * stage) */
-  const bool upd = !(mode == MODE_RHS || PART != PART_FUSED);
+  const bool upd = !(la.mode == MODE_RHS || PART != PART_FUSED);
   /* a 2N-storage scheme starts every step with A = 0 (dq = dt L): the old
    * dq is not read then */
   const bool rd_dq = upd && cx.a != 0.0;
@@ -536,7 +536,7 @@ __device__ __forceinline__ void elastic_task(const SD &sd, const Task &tk,
   /* ---- point source and manufactured forcing ---- */
   if (PART != PART_SURFACE && e == sd.src_elem)
   {
-    const TC g = (TC)cx.g;
+    const TC g = (TC)stage_g(cx, la);
     const TC w = src_tab<TC>(sd)[n];
 #pragma unroll
     for (int f = 0; f < NF; ++f)
@@ -547,7 +547,7 @@ __device__ __forceinline__ void elastic_task(const SD &sd, const Task &tk,
     const TC *T = smms + le * 6 * n1;
     const TC Sv[3] = {T[0 * n1 + i], T[2 * n1 + j], T[4 * n1 + k]};
     const TC Cv[3] = {T[1 * n1 + i], T[3 * n1 + j], T[5 * n1 + k]};
-    const TC sw = (TC)cx.sw, cw = (TC)cx.cw;
+    const TC sw = (TC)stage_sw(cx, la), cw = (TC)stage_cw(cx, la);
 #pragma unroll
     for (int f = 0; f < NF; ++f)
       rate[f] += (TC)sd.mms_F[f] * mms_pattern<TC>(f, Sv, Cv) * (f < 3 ? sw : cw);
@@ -696,7 +696,7 @@ elastic_stage_kernel(LaunchArgs a)
         const StageCtx cx = stage_ctx(sd, a);
         tk.e0 += s0;
         tk.ne = tk.ne - s0 < EPB ? tk.ne - s0 : EPB;
-        elastic_task<N, EPB, P>(sd, tk, cx, a.mode, smem);
+        elastic_task<N, EPB, P>(sd, tk, cx, a, smem);
         __syncthreads();
       }
     }
@@ -709,7 +709,7 @@ elastic_stage_kernel(LaunchArgs a)
     const StageCtx cx = stage_ctx(sd, a);
     if constexpr (EPB == TE)
     {
-      elastic_task<N, EPB, P>(sd, tk, cx, a.mode, smem);
+      elastic_task<N, EPB, P>(sd, tk, cx, a, smem);
       __syncthreads();
     }
     else
@@ -718,7 +718,7 @@ elastic_stage_kernel(LaunchArgs a)
         Task pt = tk;
         pt.e0 = tk.e0 + s0;
         pt.ne = tk.ne - s0 < EPB ? tk.ne - s0 : EPB;
-        elastic_task<N, EPB, P>(sd, pt, cx, a.mode, smem);
+        elastic_task<N, EPB, P>(sd, pt, cx, a, smem);
         __syncthreads();
       }
   }
@@ -827,7 +827,7 @@ elastic_part_kernel(LaunchArgs a)
     const Task tk = load_task(a.tasks, ti);
     const auto &sd = *(cglob(a.subs) + tk.sub);
     const StageCtx cx = stage_ctx(sd, a);
-    elastic_task<N, EPB, P64, PART>(sd, tk, cx, a.mode, smem);
+    elastic_task<N, EPB, P64, PART>(sd, tk, cx, a, smem);
     __syncthreads();
   }
 }

@@ -171,7 +171,7 @@ __device__ __forceinline__ void fold(int c, TC q, TC g, TC glam, TC gl2m,
 template <int N, class P, int PART = PART_FUSED, class SD>
 __device__ __forceinline__ void elastic_line_task(const SD &sd,
                                                   const Task &tk,
-                                                  const StageCtx &cx, int mode,
+                                                  const StageCtx &cx, const LaunchArgs &la,
                                                   char *lds, bool rows_ready,
                                                   const NextRows<typename P::TS> &nx)
 {
@@ -396,7 +396,7 @@ __device__ __forceinline__ void elastic_line_task(const SD &sd,
         }
       }
   }
-  const bool rhs_out = (mode == MODE_RHS || PART != PART_FUSED);
+  const bool rhs_out = (la.mode == MODE_RHS || PART != PART_FUSED);
   const TR ca = (TR)cx.a, cdt = (TR)cx.dt;
   const TS cb = (TS)cx.b;
   constexpr int PD = sizeof(TS) == 4 ? NF : 3;
@@ -610,7 +610,7 @@ __device__ __forceinline__ void elastic_line_task(const SD &sd,
   pass(std::integral_constant<int, 0>{}, nbx);
   /* sigma_11 is read by nothing after the x pass but the update: keep this
    * lane's row values of it and free its region for the transposes */
-  const bool keep_s11 = q_from_lds && !(mode == MODE_RHS || PART != PART_FUSED);
+  const bool keep_s11 = q_from_lds && !(la.mode == MODE_RHS || PART != PART_FUSED);
   TL s11[ROWS][VW];
   if (keep_s11)
   {
@@ -647,7 +647,7 @@ __device__ __forceinline__ void elastic_line_task(const SD &sd,
   if (act && PART != PART_SURFACE && e == sd.src_elem)
   {
     gptr<const TC> w = src_tab<TC>(sd) + n1 * L;
-    const TC g = (TC)cx.g;
+    const TC g = (TC)stage_g(cx, la);
 #pragma unroll
     for (int f = 0; f < NF; ++f)
     {
@@ -660,7 +660,7 @@ __device__ __forceinline__ void elastic_line_task(const SD &sd,
   if (act && PART != PART_SURFACE && sd.mms)
   {
     gptr<const TC> T = mms_tab<TC>(sd) + (size_t)e * 6 * n1;
-    const TC sw = (TC)cx.sw, cw = (TC)cx.cw;
+    const TC sw = (TC)stage_sw(cx, la), cw = (TC)stage_cw(cx, la);
     const TC Sy = T[2 * n1 + pa], Cy = T[3 * n1 + pa];
     const TC Sz = T[4 * n1 + pb], Cz = T[5 * n1 + pb];
 #pragma unroll
@@ -859,7 +859,7 @@ __attribute__((amdgpu_waves_per_eu(LineWaves<N, P>::value))) void elastic_line_k
       nx.e0 = nt.e0;
       nx.ne = nt.ne;
     }
-    elastic_line_task<N, P, PART>(sd, tk, cx, a.mode, mine, ready, nx);
+    elastic_line_task<N, P, PART>(sd, tk, cx, a, mine, ready, nx);
     ready = nx.valid;
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
@@ -893,11 +893,11 @@ __global__ __launch_bounds__(64 * LINE_WPB) void elastic_line_mixed(LaunchArgs a
     nx.e0 = nx.ne = 0;
     switch (tk.N)
     {
-    case 3: elastic_line_task<3, P>(sd, tk, cx, a.mode, mine, false, nx); break;
-    case 4: elastic_line_task<4, P>(sd, tk, cx, a.mode, mine, false, nx); break;
-    case 5: elastic_line_task<5, P>(sd, tk, cx, a.mode, mine, false, nx); break;
-    case 6: elastic_line_task<6, P>(sd, tk, cx, a.mode, mine, false, nx); break;
-    default: elastic_line_task<7, P>(sd, tk, cx, a.mode, mine, false, nx); break;
+    case 3: elastic_line_task<3, P>(sd, tk, cx, a, mine, false, nx); break;
+    case 4: elastic_line_task<4, P>(sd, tk, cx, a, mine, false, nx); break;
+    case 5: elastic_line_task<5, P>(sd, tk, cx, a, mine, false, nx); break;
+    case 6: elastic_line_task<6, P>(sd, tk, cx, a, mine, false, nx); break;
+    default: elastic_line_task<7, P>(sd, tk, cx, a, mine, false, nx); break;
     }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
