@@ -496,13 +496,13 @@ class Subdomain:
         _check(lib().bfamx_set_fields(self.h, _ptrs(rows), float(t0), float(dt)))
 
     def download(self):
-        q = np.zeros((self.nf, self.K * self.Np))
+        q = np.empty((self.nf, self.K * self.Np))
         rows = [q[f] for f in range(self.nf)]
         _check(lib().bfamx_download_fields(self.h, _ptrs(rows)))
         return q
 
     def rhs(self, t=0.0):
-        out = np.zeros((self.nf, self.K * self.Np))
+        out = np.empty((self.nf, self.K * self.Np))
         rows = [out[f] for f in range(self.nf)]
         _check(lib().bfamx_rhs(self.h, float(t), _ptrs(rows)))
         return out
@@ -510,7 +510,7 @@ class Subdomain:
     def rhs_noalloc(self, t=0.0):
         """bfamx_rhs_noalloc: the RHS staged in the library's fixed device
         array instead of a buffer allocated on first use"""
-        out = np.zeros((self.nf, self.K * self.Np))
+        out = np.empty((self.nf, self.K * self.Np))
         rows = [out[f] for f in range(self.nf)]
         _check(lib().bfamx_rhs_noalloc(self.h, float(t), _ptrs(rows)))
         return out
@@ -595,7 +595,7 @@ class Batch:
 
     def rhs(self, t=0.0):
         """L(q, t) of every member: list of (nfields, K*Np) arrays"""
-        outs = [np.zeros((s.nf, s.K * s.Np)) for s in self.subs]
+        outs = [np.empty((s.nf, s.K * s.Np)) for s in self.subs]
         rows = [_ptrs([o[f] for f in range(o.shape[0])]) for o in outs]
         arr = (C.c_void_p * len(rows))(*[C.cast(r, C.c_void_p) for r in rows])
         _check(lib().bfamx_batch_rhs(self.h, float(t), arr))

@@ -69,6 +69,8 @@ hipError_t launch_plain_update(const SubDev *sd_dev, int slot, size_t ndof,
 /* advance the clocks of nsubs device descriptors by m stages and refill the
  * stage parameters from slot `first` on */
 hipError_t launch_clock_advance(const SubDev *subs, int nsubs, int m, int first, hipStream_t s);
+/* set one descriptor's clock to the start of a step at t0 with step dt */
+hipError_t launch_clock_set(const SubDev *sub, double t0, double dt, hipStream_t s);
 hipError_t launch_mortar(int prec, const GlueArgs &a, hipStream_t s);
 
 /* field transfer between adapted meshes: one source or destination

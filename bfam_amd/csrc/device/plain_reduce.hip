@@ -31,37 +31,14 @@ __global__ __launch_bounds__(256) void plain_update_kernel(const SubDev *sdp, in
   }
 }
 
-/* One wavefront per subdomain: advance its clock past the m stages just run
- * and write the parameters of the next CLOCK_SLOTS stages, lane i those of
- * the i-th, from slot `first` on.  It runs after the stage kernels, so no
- * block of a stage reads the clock while it changes.  Time advances by one
- * addition of dt per step, in each lane, so that it has the same bits
- * however the stages were divided into runs. */
-__global__ __launch_bounds__(64) void clock_advance_kernel(const SubDev *subs, int m, int first)
+/* Parameters of the i-th stage from the one that is stage s of a step that
+ * starts at t, `st` stages after the first (one lane).  Time advances by one
+ * addition of dt per step, so that it has the same bits however the stages
+ * were divided into runs. */
+__device__ __forceinline__ void clock_slot(const SubDev &sd, int i, long long st, int s, double t,
+                                           double dt)
 {
-  const SubDev &sd = *(const SubDev *)(glob(subs) + blockIdx.x);
-  gptr<Clock> c = glob(sd.clock);
-  const int i = threadIdx.x, S = sd.nstages;
-  const long long st0 = c->stage;
-  const double dt = c->dt;
-  double t = c->t;
-  int s = (int)(st0 % S); /* stage within the step */
-  for (int k = 0; k < m; ++k)
-    if (++s == S)
-    {
-      s = 0;
-      t = t + dt;
-    }
-  const int s0 = s;
-  const double t0 = t;
-  __syncthreads(); /* every lane has read the clock */
-  if (i == 0)
-  {
-    c->stage = st0 + m;
-    c->t = t0;
-  }
-  if (i < first || i >= CLOCK_SLOTS)
-    return;
+  const int S = sd.nstages;
   for (int k = 0; k < i; ++k)
     if (++s == S)
     {
@@ -69,7 +46,7 @@ __global__ __launch_bounds__(64) void clock_advance_kernel(const SubDev *subs, i
       t = t + dt;
     }
   gptr<StageSlot> x = glob((StageSlot *)sd.clock->ctx) + i;
-  x->parity = (int)((st0 + m + i) & 1);
+  x->parity = (int)((st + i) & 1);
   x->dq_dead = s == S - 1 && sd.A[0] == 0.0;
   x->rec = sd.dq_rec;
   x->a = sd.AB[s];
@@ -85,6 +62,56 @@ __global__ __launch_bounds__(64) void clock_advance_kernel(const SubDev *subs, i
     x->sw = sv;
     x->cw = cv;
   }
+}
+
+/* One wavefront per subdomain: advance its clock past the m stages just run
+ * and write the parameters of the next CLOCK_SLOTS stages, lane i those of
+ * the i-th, from slot `first` on.  It runs after the stage kernels, so no
+ * block of a stage reads the clock while it changes. */
+__global__ __launch_bounds__(64) void clock_advance_kernel(const SubDev *subs, int m, int first)
+{
+  const SubDev &sd = *(const SubDev *)(glob(subs) + blockIdx.x);
+  gptr<Clock> c = glob(sd.clock);
+  const int i = threadIdx.x, S = sd.nstages;
+  const long long st = c->stage + m;
+  const double dt = c->dt;
+  double t = c->t;
+  int s = (int)(c->stage % S); /* stage within the step */
+  for (int k = 0; k < m; ++k)
+    if (++s == S)
+    {
+      s = 0;
+      t = t + dt;
+    }
+  __syncthreads(); /* every lane has read the clock */
+  if (i == 0)
+  {
+    c->stage = st;
+    c->t = t;
+  }
+  if (i >= first && i < CLOCK_SLOTS)
+    clock_slot(sd, i, st, s, t, dt);
+}
+
+/* one wavefront: a clock at the start of a step at t, no stage run */
+__global__ __launch_bounds__(64) void clock_set_kernel(const SubDev *sub, double t, double dt)
+{
+  const SubDev &sd = *(const SubDev *)glob(sub);
+  gptr<Clock> c = glob(sd.clock);
+  if (threadIdx.x == 0)
+  {
+    c->t = t;
+    c->dt = dt;
+    c->stage = 0;
+  }
+  if (threadIdx.x < CLOCK_SLOTS)
+    clock_slot(sd, threadIdx.x, 0, 0, t, dt);
+}
+
+hipError_t launch_clock_set(const SubDev *sub, double t0, double dt, hipStream_t s)
+{
+  hipLaunchKernelGGL(clock_set_kernel, dim3(1), dim3(64), 0, s, sub, t0, dt);
+  return hipGetLastError();
 }
 
 hipError_t launch_clock_advance(const SubDev *subs, int nsubs, int m, int first, hipStream_t s)

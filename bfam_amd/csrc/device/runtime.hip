@@ -19,12 +19,62 @@
 
 #include <algorithm>
 #include <atomic>
+#include <mutex>
+#include <system_error>
+#include <thread>
 #include <vector>
 
 #include "../bfamx_internal.h"
 #include "launch.hpp"
 
 using namespace bfamx;
+
+/* Staging of host field arrays (bfamx_set_fields, bfamx_download_fields,
+ * bfamx_rhs): FC_WORKERS pinned buffers of FC_BYTES, allocated with the first
+ * copy and held until bfamx_device_destroy, each with a stream of its own.
+ * One copy at a time uses them (mu). */
+constexpr int FC_WORKERS = 8;
+constexpr size_t FC_BYTES = (size_t)2 << 20;
+struct FieldCopy
+{
+  std::mutex mu;
+  char *buf[FC_WORKERS] = {};
+  bool pinned[FC_WORKERS] = {};
+  hipStream_t st[FC_WORKERS] = {};
+  /* the buffer and stream of worker i */
+  hipError_t get(int i)
+  {
+    if (!buf[i])
+    {
+      void *p = NULL;
+      pinned[i] = hipHostMalloc(&p, FC_BYTES, hipHostMallocDefault) == hipSuccess;
+      if (!pinned[i])
+      {
+        (void)hipGetLastError();
+        p = malloc(FC_BYTES);
+      }
+      if (!p)
+        return hipErrorOutOfMemory;
+      buf[i] = (char *)p;
+    }
+    return st[i] ? hipSuccess : hipStreamCreateWithFlags(&st[i], hipStreamNonBlocking);
+  }
+  ~FieldCopy()
+  {
+    for (int i = 0; i < FC_WORKERS; ++i)
+    {
+      if (st[i])
+      {
+        (void)hipStreamSynchronize(st[i]);
+        (void)hipStreamDestroy(st[i]);
+      }
+      if (pinned[i])
+        (void)hipHostFree(buf[i]);
+      else
+        free(buf[i]);
+    }
+  }
+};
 
 struct bfamx_device
 {
@@ -70,6 +120,7 @@ struct bfamx_device
   hipEvent_t fork_ev, join_ev[8];
   /* device address of this GPU's copy of `scratch` (bfamx_rhs_noalloc) */
   double *scratch;
+  FieldCopy fc;
 };
 
 /* Staging buffer of bfamx_rhs_noalloc: one copy per GPU, held until the
@@ -485,6 +536,14 @@ static int refresh_clock(bfamx_subdomain_t *s)
 {
   s->clock_by = 0;
   HIPCHK(launch_clock_advance(s->d_sub, 1, 0, 0, s->dev->stream));
+  return BFAMX_OK;
+}
+
+/* start the clock at t0 with step dt, no stage run */
+static int set_clock(bfamx_subdomain_t *s, double t0, double dt)
+{
+  s->clock_by = 0;
+  HIPCHK(launch_clock_set(s->d_sub, t0, dt, s->dev->stream));
   return BFAMX_OK;
 }
 
@@ -914,6 +973,117 @@ extern "C" int bfamx_set_forcing_mms(bfamx_subdomain_t *s, double k,
   return refresh_clock(s);
 }
 
+/* elements [e0, e1) of a [K][nf][Np] array of T (buf: from e0 on) to or from
+ * bfam's per-field host arrays */
+template <class T, bool OUT, class F>
+static void host_rows(T *buf, F *const *fields, size_t e0, size_t e1, size_t nf, size_t Np)
+{
+  for (size_t f = 0; f < nf; ++f)
+    for (size_t e = e0; e < e1; ++e)
+    {
+      T *b = buf + ((e - e0) * nf + f) * Np;
+      F *h = fields[f] + e * Np;
+      if constexpr (OUT)
+        for (size_t n = 0; n < Np; ++n)
+          h[n] = (double)b[n];
+      else
+        for (size_t n = 0; n < Np; ++n)
+          b[n] = (T)h[n];
+    }
+}
+
+/*
+ * A device [K][nf][Np] array of T to (OUT) or from the host's per-field
+ * double arrays.  The array moves in pieces of whole elements through pinned
+ * buffers; a large one is divided over up to FC_WORKERS host threads, each
+ * with its own buffer and stream, so that one thread's transfer runs under
+ * another's conversion and the first touches of the caller's pages are
+ * spread.  Work of the device's stream issued before is complete when a
+ * copy out starts, and before a copy in starts the caller has synchronised.
+ * A single unpinned buffer converted by one thread took 212 ms out for a 32^3
+ * N=7 FP32 state (1.2 GB of doubles; here 25 ms).
+ */
+template <class T, bool OUT, class F>
+static int copy_fields(bfamx_subdomain_t *s, void *dev_array, F *const *fields)
+{
+  bfamx_device_t *d = s->dev;
+  const size_t Np = s->Np, nf = s->nf, K = s->K;
+  const size_t per = nf * Np * sizeof(T), total = K * per;
+  std::lock_guard<std::mutex> lock(d->fc.mu);
+  /* one worker per 512 KiB, pieces of at least 256 KiB (at most 2 MiB, a
+   * buffer) so that each worker has two or more */
+  const size_t want = total / ((size_t)512 << 10);
+  const int nw = want < 2 ? 1 : want < FC_WORKERS ? (int)want : FC_WORKERS;
+  size_t bytes = total / (2 * nw);
+  bytes = bytes < ((size_t)256 << 10) ? (size_t)256 << 10 : bytes > FC_BYTES ? FC_BYTES : bytes;
+  if (nw == 1)
+    bytes = FC_BYTES;
+  const size_t kc = std::max<size_t>(1, bytes / per);
+  int dev0 = 0; /* the buffers and streams belong to this device */
+  HIPCHK(hipGetDevice(&dev0));
+  hipError_t ge = hipSetDevice(d->hip_dev);
+  for (int i = 0; i < nw && ge == hipSuccess; ++i)
+    ge = d->fc.get(i);
+  (void)hipSetDevice(dev0);
+  HIPCHK(ge);
+  std::atomic<size_t> next{0};
+  std::atomic<int> err{hipSuccess};
+  auto work = [&](int w, hipStream_t st) {
+    T *buf = (T *)d->fc.buf[w];
+    for (size_t e0 = next.fetch_add(kc); e0 < K && err == hipSuccess; e0 = next.fetch_add(kc))
+    {
+      const size_t e1 = std::min(K, e0 + kc);
+      T *dev = (T *)dev_array + e0 * nf * Np;
+      const size_t nb = (e1 - e0) * per;
+      if constexpr (!OUT)
+        host_rows<T, OUT>(buf, fields, e0, e1, nf, Np);
+      hipError_t e = OUT ? hipMemcpyAsync(buf, dev, nb, hipMemcpyDeviceToHost, st)
+                         : hipMemcpyAsync(dev, buf, nb, hipMemcpyHostToDevice, st);
+      if (e == hipSuccess)
+        e = hipStreamSynchronize(st);
+      if (e != hipSuccess)
+      {
+        err = e;
+        return;
+      }
+      if constexpr (OUT)
+        host_rows<T, OUT>(buf, fields, e0, e1, nf, Np);
+    }
+  };
+  if (nw == 1)
+    work(0, d->stream);
+  else
+  {
+    HIPCHK(hipStreamSynchronize(d->stream));
+    std::vector<std::thread> th;
+    th.reserve(nw);
+    for (int i = 1; i < nw; ++i)
+    {
+      try
+      {
+        th.emplace_back([&, i] {
+          const hipError_t e = hipSetDevice(d->hip_dev);
+          if (e != hipSuccess)
+            err = e;
+          else
+            work(i, d->fc.st[i]);
+        });
+      }
+      catch (const std::system_error &)
+      {
+        break; /* no more threads: those that run take the pieces */
+      }
+    }
+    work(0, d->fc.st[0]);
+    for (std::thread &t : th)
+      t.join();
+  }
+  if (err != hipSuccess)
+    return bfamx_fail(BFAMX_EHIP, "field copy failed: %s",
+                      hipGetErrorString((hipError_t)err.load()));
+  return BFAMX_OK;
+}
+
 extern "C" int bfamx_set_fields(bfamx_subdomain_t *s,
                                 const double *const *fields, double t0,
                                 double dt)
@@ -924,48 +1094,33 @@ extern "C" int bfamx_set_fields(bfamx_subdomain_t *s,
     for (int f = 0; f < s->nf; ++f)
       if (!fields[f])
         return bfamx_fail(BFAMX_EINVAL, "bfamx_set_fields: field %d is NULL", f);
-  const size_t Np = s->Np, nf = s->nf, K = s->K;
-  const size_t ndof = K * nf * Np;
-  HIPCHK(hipStreamSynchronize(s->dev->stream));
+  const size_t ndof = (size_t)s->K * s->nf * s->Np;
+  hipStream_t st = s->dev->stream;
+  HIPCHK(hipStreamSynchronize(st));
+  int rc = BFAMX_OK;
   if (!fields)
-    HIPCHK(hipMemset(s->h.q[0], 0, (s->state_fp32 ? 4 : 8) * ndof));
-  else if (s->state_fp32)
-  {
-    std::vector<float> buf(ndof);
-    for (size_t e = 0; e < K; ++e)
-      for (size_t f = 0; f < nf; ++f)
-        for (size_t n = 0; n < Np; ++n)
-          buf[(e * nf + f) * Np + n] = (float)fields[f][e * Np + n];
-    HIPCHK(hipMemcpy(s->h.q[0], buf.data(), 4 * ndof, hipMemcpyHostToDevice));
-  }
+    HIPCHK(hipMemsetAsync(s->h.q[0], 0, (s->state_fp32 ? 4 : 8) * ndof, st));
   else
-  {
-    std::vector<double> buf(ndof);
-    for (size_t e = 0; e < K; ++e)
-      for (size_t f = 0; f < nf; ++f)
-        for (size_t n = 0; n < Np; ++n)
-          buf[(e * nf + f) * Np + n] = fields[f][e * Np + n];
-    HIPCHK(hipMemcpy(s->h.q[0], buf.data(), 8 * ndof, hipMemcpyHostToDevice));
-  }
+    rc = s->state_fp32 ? copy_fields<float, false>(s, s->h.q[0], fields)
+                       : copy_fields<double, false>(s, s->h.q[0], fields);
+  if (rc)
+    return rc;
   if (s->h.dq)
-    HIPCHK(hipMemset(s->h.dq, 0, (s->rate_fp32 ? 4 : 8) * ndof));
-  const ClockHead c = {t0, dt, 0};
-  HIPCHK(hipMemcpy(s->d_clock, &c, sizeof(c), hipMemcpyHostToDevice));
+    HIPCHK(hipMemsetAsync(s->h.dq, 0, (s->rate_fp32 ? 4 : 8) * ndof, st));
+  rc = set_clock(s, t0, dt);
+  if (rc)
+    return rc;
   s->fields_set = 1;
   s->t0_set = t0;
   s->dt_set = dt;
   s->stages_run = 0;
-  return refresh_clock(s);
+  return BFAMX_OK;
 }
 
-static int current_parity(bfamx_subdomain_t *s, int *parity)
+/* which buffer holds the state after the stages launched so far */
+static int current_parity(const bfamx_subdomain_t *s)
 {
-  ClockHead c;
-  int rc = read_clock(s, &c);
-  if (rc)
-    return rc;
-  *parity = s->prec == BFAMX_FP64_PLAIN ? 0 : (int)(c.stage & 1);
-  return BFAMX_OK;
+  return s->prec == BFAMX_FP64_PLAIN ? 0 : (int)(s->stages_run & 1);
 }
 
 extern "C" int bfamx_get_time(bfamx_subdomain_t *s, double *t, int64_t *stages)
@@ -983,21 +1138,6 @@ extern "C" int bfamx_get_time(bfamx_subdomain_t *s, double *t, int64_t *stages)
   return BFAMX_OK;
 }
 
-/* copy a device [K][nf][Np] array of T into bfam's per-field host layout */
-template <class T>
-static int download_layout(const bfamx_subdomain_t *s, const void *src,
-                           double *const *fields)
-{
-  const size_t Np = s->Np, nf = s->nf, K = s->K;
-  std::vector<T> buf(K * nf * Np);
-  HIPCHK(hipMemcpy(buf.data(), src, sizeof(T) * buf.size(), hipMemcpyDeviceToHost));
-  for (size_t e = 0; e < K; ++e)
-    for (size_t f = 0; f < nf; ++f)
-      for (size_t n = 0; n < Np; ++n)
-        fields[f][e * Np + n] = (double)buf[(e * nf + f) * Np + n];
-  return BFAMX_OK;
-}
-
 extern "C" int bfamx_download_fields(bfamx_subdomain_t *s,
                                      double *const *fields)
 {
@@ -1005,11 +1145,9 @@ extern "C" int bfamx_download_fields(bfamx_subdomain_t *s,
     return bfamx_fail(BFAMX_EINVAL, "bfamx_download_fields: NULL argument");
   if (!s->fields_set)
     return bfamx_fail(BFAMX_ESTATE, "bfamx_download_fields: no state set");
-  int parity, rc = current_parity(s, &parity);
-  if (rc)
-    return rc;
-  return s->state_fp32 ? download_layout<float>(s, s->h.q[parity], fields)
-                       : download_layout<double>(s, s->h.q[parity], fields);
+  const int parity = current_parity(s);
+  return s->state_fp32 ? copy_fields<float, true>(s, s->h.q[parity], fields)
+                       : copy_fields<double, true>(s, s->h.q[parity], fields);
 }
 
 static LaunchArgs launch_args(bfamx_subdomain_t *s, int mode)
@@ -1341,8 +1479,7 @@ static int rhs_one(bfamx_subdomain_t *s, double t, double *const *rhs)
   rc = rhs_launch(s, t);
   if (rc)
     return rc;
-  HIPCHK(hipStreamSynchronize(s->dev->stream));
-  return download_layout<double>(s, s->h.rhs, rhs);
+  return copy_fields<double, true>(s, s->h.rhs, rhs);
 }
 
 /* Neumaier's compensated sum of n values with stride */
@@ -1366,10 +1503,7 @@ extern "C" int bfamx_reduce_energy(bfamx_subdomain_t *s, double *energy)
 {
   if (!s || !energy)
     return bfamx_fail(BFAMX_EINVAL, "bfamx_reduce_energy: NULL argument");
-  int parity, rc = current_parity(s, &parity);
-  if (rc)
-    return rc;
-  hipError_t e = launch_energy(s->h, s->state_fp32, parity, s->d_partial,
+  hipError_t e = launch_energy(s->h, s->state_fp32, current_parity(s), s->d_partial,
                                s->dev->stream);
   if (e != hipSuccess)
     return bfamx_fail(BFAMX_EHIP, "energy launch: %s", hipGetErrorString(e));
@@ -1405,10 +1539,8 @@ extern "C" int bfamx_reduce_l2_diff(bfamx_subdomain_t *a, bfamx_subdomain_t *b,
     return bfamx_fail(BFAMX_EINVAL, "bfamx_reduce_l2_diff: NULL argument");
   if (a->K != b->K || a->N != b->N || a->physics != b->physics || a->dev != b->dev)
     return bfamx_fail(BFAMX_EINVAL, "bfamx_reduce_l2_diff: different shapes");
-  int pa, pb, rc = current_parity(a, &pa);
-  if (rc || (rc = current_parity(b, &pb)))
-    return rc;
-  hipError_t e = launch_l2diff(a->h, a->state_fp32, pa, b->h, b->state_fp32, pb,
+  hipError_t e = launch_l2diff(a->h, a->state_fp32, current_parity(a), b->h, b->state_fp32,
+                               current_parity(b),
                                a->d_partial, a->dev->stream);
   if (e != hipSuccess)
     return bfamx_fail(BFAMX_EHIP, "l2diff launch: %s", hipGetErrorString(e));
@@ -2305,12 +2437,9 @@ extern "C" int bfamx_batch_autotune(bfamx_batch_t *b, int trials, int force,
     reg[i] = s->h.dq;
     if (s->h.dq_rec)
     {
-      int parity = 0;
-      rc = current_parity(s, &parity);
-      reg[i] = s->h.q[parity ^ 1];
+      reg[i] = s->h.q[current_parity(s) ^ 1];
     }
-    if (!rc)
-      rc = dev_alloc(d, allocs, &bytes, nb, &saved[i]);
+    rc = dev_alloc(d, allocs, &bytes, nb, &saved[i]);
     if (!rc && hipMemcpyAsync(saved[i], reg[i], nb, hipMemcpyDeviceToDevice, d->stream) !=
                    hipSuccess)
       rc = bfamx_fail(BFAMX_EHIP, "autotune: dq save failed");
@@ -2655,10 +2784,7 @@ extern "C" int bfamx_transfer_fields(const bfamx_transfer_maps_t *m,
   std::vector<XferSide> hs(nsrc), hd(ndst);
   for (int i = 0; i < nsrc; ++i)
   {
-    int parity = 0, rc = current_parity(src[i], &parity);
-    if (rc)
-      return rc;
-    hs[i].q = src[i]->h.q[parity];
+    hs[i].q = src[i]->h.q[current_parity(src[i])];
     hs[i].N = src[i]->N;
     hs[i].K = src[i]->K;
   }
@@ -2714,16 +2840,14 @@ extern "C" int bfamx_transfer_fields(const bfamx_transfer_maps_t *m,
     bfamx_subdomain_t *s = dst[i];
     const size_t ndof = (size_t)s->K * s->nf * s->Np;
     if (s->h.dq)
-      HIPCHK(hipMemset(s->h.dq, 0, (s->rate_fp32 ? 4 : 8) * ndof));
-    const ClockHead c = {t, dt, 0};
-    HIPCHK(hipMemcpy(s->d_clock, &c, sizeof(c), hipMemcpyHostToDevice));
+      HIPCHK(hipMemsetAsync(s->h.dq, 0, (s->rate_fp32 ? 4 : 8) * ndof, dev->stream));
+    rc = set_clock(s, t, dt);
+    if (rc)
+      return rc;
     s->fields_set = 1;
     s->t0_set = t;
     s->dt_set = dt;
     s->stages_run = 0;
-    rc = refresh_clock(s);
-    if (rc)
-      return rc;
   }
   return BFAMX_OK;
 }
