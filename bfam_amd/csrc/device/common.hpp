@@ -312,48 +312,42 @@ __device__ __forceinline__ size_t qidx(int e, int f, int n, int NF, int Np)
 }
 
 /*
- * Order in which a block walks the task list.  Hardware dispatches
- * consecutive workgroups round-robin over the XCDs.  Mode 0 keeps that
- * order; mode 1 gives XCD x the contiguous slice [x*C, (x+1)*C) of the
- * (Morton-ordered) task list; mode 2 (the default) keeps one round-robin
- * front over the list but hands each XCD whole 2x2x2 Morton cubes.
+ * Order in which a block walks n tasks: task_at(v) for v = first, first +
+ * stride, .. below end.  Hardware dispatches consecutive workgroups
+ * round-robin over the XCDs.  Mode 0 keeps that order; mode 1 gives XCD x
+ * the contiguous slice [x*C, (x+1)*C) of the (Morton-ordered) task list; mode
+ * 2 (the default) keeps one round-robin front over the list but hands each
+ * XCD whole Morton cubes of XC tasks, whose inner faces then share an L2.
  */
-__device__ __forceinline__ int first_task(const LaunchArgs &a, int ntasks, int *stride,
-                                          int *end)
+struct TaskWalk
+{
+  int first, stride, end;
+};
+__device__ __forceinline__ TaskWalk task_walk(const LaunchArgs &a, int n)
 {
   const int b = blockIdx.x, G = gridDim.x;
-  if (a.xcd_remap == 2 && a.nxcd == 8 && G >= ntasks)
-  {
-    /* round-robin front, but each XCD's 8 blocks of a group of 64 take one
-     * 2x2x2 Morton cube of tasks, whose inner faces then share an L2; a
-     * partial last group keeps the identity */
-    *stride = G;
-    *end = ntasks;
-    const int g0 = b & ~63;
-    if (g0 + 64 > ntasks)
-      return b;
-    return g0 + 8 * (b & 7) + ((b & 63) >> 3);
-  }
   if (a.xcd_remap != 1 || G % a.nxcd)
-  {
-    *stride = G;
-    *end = ntasks;
-    return b;
-  }
-  const int x = b % a.nxcd, s = b / a.nxcd, per = G / a.nxcd;
-  const int C = (ntasks + a.nxcd - 1) / a.nxcd;
-  const int lo = x * C;
-  int hi = lo + C;
-  if (hi > ntasks)
-    hi = ntasks;
-  *stride = per;
-  *end = hi;
-  return lo + s;
+    return {b, G, n};
+  const int x = b % a.nxcd, s = b / a.nxcd, C = (n + a.nxcd - 1) / a.nxcd;
+  const int lo = x * C, hi = lo + C;
+  return {lo + s, G / a.nxcd, hi < n ? hi : n};
 }
-
-__device__ __forceinline__ int first_task(const LaunchArgs &a, int *stride, int *end)
+/* a grid whose blocks keep their XCD over the walk: every task its own
+ * block, or a multiple of the XCDs */
+template <int XC = 8>
+__device__ __forceinline__ int task_at(const LaunchArgs &a, int n, int v)
 {
-  return first_task(a, a.ntasks, stride, end);
+  if (a.xcd_remap != 2 || a.nxcd != 8 || ((int)gridDim.x < n && gridDim.x % 8))
+    return v;
+  /* the XC blocks of each XCD in a group of 8 XC take one cube; of the
+   * partial last group, cubes of 8 as far as they go, then the identity */
+  const int g0 = v & ~(8 * XC - 1);
+  if (g0 + 8 * XC <= n)
+    return g0 + XC * (v & 7) + ((v & (8 * XC - 1)) >> 3);
+  const int g1 = v & ~63;
+  if (g1 + 64 > n)
+    return v;
+  return g1 + 8 * (v & 7) + ((v & 63) >> 3);
 }
 
 /* Ricker wavelet (1 - 2a) exp(-a), a = (pi f0 (t - t0))^2 */

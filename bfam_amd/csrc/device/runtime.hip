@@ -246,9 +246,9 @@ extern "C" int bfamx_device_create(int hip_device, size_t hbm_budget_bytes,
     nx = 1;
   d->num_xcd = nx;
   /* block order: one round-robin front over the elements, each XCD taking
-   * whole 2x2x2 Morton cubes (48^3 N=7 stage: FP32 1.48 ms, against 1.50
-   * for the plain round-robin order and 1.55 for contiguous XCD slices;
-   * FP64 2.79, 2.87 and 2.99 ms) */
+   * whole Morton cubes (48^3 N=7 stage with 2x2x2 cubes: FP32 1.48 ms,
+   * against 1.50 for the plain round-robin order and 1.55 for contiguous
+   * XCD slices; FP64 2.79, 2.87 and 2.99 ms; NODE_XC for the cubes' size) */
   d->xcd_remap = 2;
   memset(d->mixed_choice, -1, sizeof(d->mixed_choice));
   d->persistent = 0;
@@ -1176,11 +1176,11 @@ static int grid_for(const bfamx_device_t *d, int ntasks)
 
 /* the stage kernel of an order not (yet) autotuned (0 line, 1
  * node-parallel, 2 node-parallel on a resident grid): the one measured
- * fastest on bricks of about 124 M DOF (FP32: resident grid at N = 4 and
- * 6, node-parallel at N = 3, 5 and 7; FP64: node-parallel at N = 3..5,
- * resident grid at N = 6, 7; at N = 5 the two node-parallel grids are
- * within 5 % of each other), and the node-parallel kernel for FP32_RHS and
- * split-BF16x3 */
+ * fastest, us per stage with one block per task / on the resident grid:
+ * FP32 N=4 78.5 / 95.0 (27^3) and 394 / 437 (46^3), N=5 316 / 333 (38^3),
+ * N=6 64.0 / 63.2 (18^3) and 346 / 325 (32^3), N=7 374 / 410 (32^3); FP64
+ * N=5 351 / 366 (32^3), N=6 91 / 82 (16^3) and 380 / 336 (26^3), N=7 90 / 101
+ * (16^3) and 374 / 420 (26^3); FP32 rates N=6 420 / 562 (28^3) */
 static int default_kind(int prec, int N)
 {
   switch (prec)

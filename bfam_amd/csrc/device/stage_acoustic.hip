@@ -222,10 +222,10 @@ __global__ __launch_bounds__(EPB *(N + 1) * (N + 1)) void
 acoustic_stage_kernel(LaunchArgs a)
 {
   __shared__ __align__(16) char smem[AcousticSmem<N, EPB, typename P::TC>::bytes];
-  int stride, end;
-  for (int ti = first_task(a, &stride, &end); ti < end; ti += stride)
+  const TaskWalk w = task_walk(a, a.ntasks);
+  for (int v = w.first; v < w.end; v += w.stride)
   {
-    const Task tk = load_task(a.tasks, ti);
+    const Task tk = load_task(a.tasks, task_at(a, a.ntasks, v));
     const auto &sd = *(cglob(a.subs) + tk.sub);
     const StageCtx cx = stage_ctx(sd, a);
     acoustic_task<N, EPB, P>(sd, tk, cx, a, smem);
@@ -276,10 +276,10 @@ __global__ __launch_bounds__(EPB *(N + 1) * (N + 1)) void
 acoustic_part_kernel(LaunchArgs a)
 {
   __shared__ __align__(16) char smem[AcousticSmem<N, EPB, double>::bytes];
-  int stride, end;
-  for (int ti = first_task(a, &stride, &end); ti < end; ti += stride)
+  const TaskWalk w = task_walk(a, a.ntasks);
+  for (int v = w.first; v < w.end; v += w.stride)
   {
-    const Task tk = load_task(a.tasks, ti);
+    const Task tk = load_task(a.tasks, task_at(a, a.ntasks, v));
     const auto &sd = *(cglob(a.subs) + tk.sub);
     const StageCtx cx = stage_ctx(sd, a);
     acoustic_task<N, EPB, P64, PART>(sd, tk, cx, a, smem);

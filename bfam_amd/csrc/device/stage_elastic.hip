@@ -34,6 +34,8 @@
  * The task, descriptor, clock and, for one-element blocks, the element
  * tables are read through the constant address space (scalar loads).
  */
+#include <type_traits>
+
 #include "elastic_axis.hpp"
 #include "mfma_deriv.hpp"
 #include "physics.hpp"
@@ -54,6 +56,45 @@ template <int N> struct NodeFaceLift
 {
   static constexpr bool value = N == 4 || N == 5 || N == 7;
   static constexpr int FC = value ? FACE_LIFT_N : 6;
+};
+
+/* How the fused kernel's face work is divided (one-element blocks).  Units:
+ * one face per wavefront (wave w takes faces w, w + W, ..), so that the
+ * face, its neighbour, its impedances and its axis are uniform in the wave
+ * (scalar loads and one flux, no select among three), and its traces are
+ * requested with the state, before the barrier.  Otherwise tasks: face nodes
+ * dealt to the threads in order, gathered after the barrier.  N = 7 has as
+ * many lanes as face nodes and eight wavefronts for its six faces; at the
+ * lower orders a unit leaves lanes idle, and the early gathers cost registers
+ * (FP32 N = 6: 69 against 64 us per 18^3 stage; N = 3: 57 against 52).  us per
+ * stage, tasks / units: N = 7 FP32 1272 / 1250 (48^3), 378 / 372 (32^3), 51.5 /
+ * 50.5 (16^3); FP64 1534 / 1420 (40^3, resident grid); FP32 rates 1350 / 1236
+ * (40^3), 95 / 86 (16^3), where FP64 traces are six loads of two registers;
+ * N = 6 FP32 rates 420 / 391 (28^3), 96 / 91 (17^3). */
+template <int N, int EPB, class P> struct NodeUnits
+{
+  static constexpr bool value =
+      EPB == 1 && !P::MF && (N == 7 || (N == 6 && __is_same(P, P32R)));
+};
+
+/* threads of a block: its volume nodes, and for face units whole wavefronts */
+template <int N, int EPB, class P> struct NodeBlock
+{
+  static constexpr int nodes = EPB * (N + 1) * (N + 1) * (N + 1);
+  static constexpr int value = NodeUnits<N, EPB, P>::value ? (nodes + 63) / 64 * 64 : nodes;
+};
+
+/* Whether a block requests its face indices and D after the state's LDS-DMA
+ * and before the barrier.  Otherwise D's round trip through a register comes
+ * before the DMA, and the index loads after the barrier, ahead of the
+ * gathers.  us per stage, later / here: FP32 N = 3 (30^3) 52.3 / 50.3, N = 5
+ * (10^3) 12.65 / 12.41 and (21^3) 58.8 / 58.8, N = 6 (18^3) 72.5 / 63.1, N = 7
+ * (32^3) 374 / 371; FP32 rates N = 3 (24^3) 42.1 / 40.4; FP64 N = 5 (18^3)
+ * 70.6 / 69.6; but FP32 N = 4 (27^3) 77.0 / 81.4, (46^3) 386 / 410. */
+template <int N, class P, bool SPLIT> struct NodeEarly
+{
+  /* the whole-task form of N = 3, at its 80 registers, would spill more */
+  static constexpr bool value = N != 4 && (N != 3 || SPLIT || !__is_same(P, P32));
 };
 
 /* the dq rows of a task are staged in LDS by LDS-DMA (no registers held
@@ -110,7 +151,7 @@ __device__ __forceinline__ void block_to_lds(gptr<const float> src, float *dst,
   }
 }
 
-template <int N, int EPB, class P, int PART = PART_FUSED, class SD>
+template <int N, int EPB, class P, int PART = PART_FUSED, bool SPLIT = false, class SD>
 __device__ __forceinline__ void elastic_task(const SD &sd, const Task &tk,
                                              const StageCtx &cx, const LaunchArgs &la,
                                              char *smem)
@@ -124,6 +165,15 @@ __device__ __forceinline__ void elastic_task(const SD &sd, const Task &tk,
   constexpr int BS = EPB * Np;
   constexpr int NT = EPB * 6 * Nfp;
   constexpr int TPT = (NT + BS - 1) / BS;
+  /* face tasks axis-major (axis, element, side, face node), so that the
+   * waves of a block mostly see faces of one axis: the flux and lift of an
+   * axis run once per wave, not once per axis present in it */
+  constexpr int TPA = EPB * 2 * Nfp;
+  constexpr int BT = NodeBlock<N, EPB, P>::value;
+  /* face units of the block's W wavefronts, R rounds of them */
+  constexpr bool UNITS = NodeUnits<N, EPB, P>::value;
+  constexpr int W = (BT + 63) / 64, R = UNITS ? (6 + W - 1) / W : 1;
+  constexpr bool EARLY = !UNITS && NodeEarly<N, P, SPLIT>::value;
   using SM = NodeSmem<N, EPB, P>;
   /* state staged exactly (FP32, FP64): LDS-DMA straight into the staged
    * fields, 16 bytes per lane.  An element's words (QE state, DE dq) are
@@ -160,24 +210,27 @@ __device__ __forceinline__ void elastic_task(const SD &sd, const Task &tk,
   TC *sD = sfl + SM::FW;
   TC *smms = sD + n1 * n1;
 
-  {
+  /* D and the sin/cos tables into LDS */
+  auto stage_tables = [&]() {
     gptr<const TC> Dg = dr_tab<TC>(sd);
     for (int t = tid; t < n1 * n1; t += blockDim.x)
       sD[t] = Dg[t];
-  }
-  if (PART != PART_SURFACE && sd.mms)
-  {
-    gptr<const TC> mt = mms_tab<TC>(sd) + (size_t)tk.e0 * 6 * n1;
-    for (int t = tid; t < tk.ne * 6 * n1; t += blockDim.x)
-      smms[t] = mt[t];
-  }
+    if (PART != PART_SURFACE && sd.mms)
+    {
+      gptr<const TC> mt = mms_tab<TC>(sd) + (size_t)tk.e0 * 6 * n1;
+      for (int t = tid; t < tk.ne * 6 * n1; t += blockDim.x)
+        smms[t] = mt[t];
+    }
+  };
+  if constexpr (!EARLY && !UNITS)
+    stage_tables();
 
   /* ---- 1. stream the element's state into LDS ---- */
   gptr<const TS> qin = glob(static_cast<const TS *>(sd.q[cx.parity]));
   TS qs[KEEP_Q ? NF : 1];
   if constexpr (DMA_Q)
   {
-    block_to_lds<16, BS>((gptr<const float>)(qin + (size_t)tk.e0 * NF * Np) - shq,
+    block_to_lds<16, BT>((gptr<const float>)(qin + (size_t)tk.e0 * NF * Np) - shq,
                          reinterpret_cast<float *>(smem), (shq + tk.ne * QE + 3) & ~3);
   }
   else if (act)
@@ -211,7 +264,7 @@ __device__ __forceinline__ void elastic_task(const SD &sd, const Task &tk,
   if constexpr (DMA_DQ)
   {
     if (rd_dq)
-      block_to_lds<16, BS, CPOL_NT>(
+      block_to_lds<16, BT, CPOL_NT>(
           (gptr<const float>)glob(static_cast<const float *>(dsrc)) + (size_t)tk.e0 * DE - shd,
           reinterpret_cast<float *>(smem + sizeof(TC) * SM::QR), (shd + tk.ne * DE + 3) & ~3);
   }
@@ -229,6 +282,73 @@ __device__ __forceinline__ void elastic_task(const SD &sd, const Task &tk,
         dqs[f] = __builtin_nontemporal_load(&dqe[f * Np]);
     }
   }
+  /* neighbour element and code of this thread's face tasks, so that after
+   * the barrier the gathers wait for no index */
+  int32_t fep[TPT];
+  int fcode[TPT];
+  if constexpr (EARLY)
+  {
+    if constexpr (PART != PART_VOLUME)
+    {
+#pragma unroll
+      for (int r = 0; r < TPT; ++r)
+      {
+        const int t = tid + r * BS;
+        const int A = t / TPA, ra = t - A * TPA;
+        const int lt = EPB == 1 ? 0 : ra / (2 * Nfp);
+        if (tid < BS && t < NT && lt < tk.ne)
+        {
+          const size_t fi = (size_t)(tk.e0 + lt) * 6 + 2 * A + (ra - lt * 2 * Nfp) / Nfp;
+          fep[r] = glob(sd.nbr_elem)[fi];
+          fcode[r] = glob(sd.nbr_code)[fi];
+        }
+      }
+    }
+    stage_tables();
+  }
+  /* units: the face's neighbour and its trace, requested with the state.
+   * The code is a byte of the table's aligned word (scalar loads are whole
+   * words; the table's allocation is a multiple of 256 bytes) */
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), fn_u = tid & 63;
+  auto unit_node = [&](int f) -> int {
+    const int a = fn_u % n1, b = fn_u / n1;
+    const int st = f < 2 ? 1 : (f < 4 ? n1 : Nfp);
+    return (f < 2 ? n1 * fn_u : (f < 4 ? a + Nfp * b : fn_u)) + ((f & 1) ? N * st : 0);
+  };
+  TS gq[R][6];
+  int32_t gep[R];
+  int gcode[R];
+  if constexpr (UNITS && PART != PART_VOLUME)
+  {
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+    {
+      const int f = wave + r * W;
+      if (f < 6 && fn_u < Nfp)
+      {
+        const size_t fi = (size_t)tk.e0 * 6 + f;
+        gep[r] = cglob(sd.nbr_elem)[fi];
+        gcode[r] = (int)(cglob((const uint32_t *)sd.nbr_code)[fi >> 2] >> (8 * (fi & 3))) & 255;
+        if (!(gcode[r] & NBR_GLUED))
+        {
+          const int A = f >> 1;
+          const int c0 = A == 0 ? sfield(0, 0) : (A == 1 ? sfield(0, 1) : sfield(0, 2));
+          const int c1 = A == 0 ? sfield(1, 0) : (A == 1 ? sfield(1, 1) : sfield(1, 2));
+          const int c2 = A == 0 ? sfield(2, 0) : (A == 1 ? sfield(2, 1) : sfield(2, 2));
+          gptr<const TS> qp =
+              qin + (size_t)gep[r] * NF * Np + nbr_node(gcode[r], f, n1, unit_node(f));
+          gq[r][0] = qp[0];
+          gq[r][1] = qp[Np];
+          gq[r][2] = qp[2 * Np];
+          gq[r][3] = qp[c0 * Np];
+          gq[r][4] = qp[c1 * Np];
+          gq[r][5] = qp[c2 * Np];
+        }
+      }
+    }
+  }
+  if constexpr (UNITS)
+    stage_tables();
   /* LDS-DMA completes by vmcnt: every wave drains its own before the
    * barrier that publishes the staged state */
   if constexpr (DMA_Q || DMA_DQ)
@@ -236,15 +356,83 @@ __device__ __forceinline__ void elastic_task(const SD &sd, const Task &tk,
   __syncthreads();
 
   /* ---- 2. faces: one task per face node, its lift values straight to LDS ---- */
-  if constexpr (PART != PART_VOLUME)
+  if constexpr (UNITS && PART != PART_VOLUME)
+  {
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+    {
+      const int f = wave + r * W;
+      if (f < 6 && fn_u < Nfp)
+      {
+        auto unit = [&](auto AX) {
+          constexpr int A = decltype(AX)::value;
+          const TC s = (f & 1) ? TC(1) : TC(-1);
+          EP Mm = (EP)mat_tab<TC>(sd) + (size_t)tk.e0 * MAT_STRIDE;
+          TC dv[3], dT[3];
+          if (gcode[r] & NBR_GLUED)
+          {
+            /* fluctuations already on this face node (mortar kernel) */
+            gptr<const TC> gb = glob(static_cast<const TC *>(sd.glue_buf)) + gep[r] + fn_u;
+#pragma unroll
+            for (int c = 0; c < 3; ++c)
+            {
+              dv[c] = gb[c * Nfp];
+              dT[c] = gb[(3 + c) * Nfp];
+            }
+          }
+          else
+          {
+            const TC *um = sq + unit_node(f);
+            TC sv, ss;
+            nbr_mirror<TC>(gcode[r], &sv, &ss);
+            TC vm[3], Sm[3], vp[3], Sp[3];
+#pragma unroll
+            for (int c = 0; c < 3; ++c)
+            {
+              vm[c] = um[c * Np];
+              Sm[c] = um[sfield(c, A) * Np];
+              vp[c] = sv * (TC)gq[r][c];
+              Sp[c] = ss * (TC)gq[r][3 + c];
+            }
+            EP F = (EP)fmat_tab<TC>(sd) + ((size_t)tk.e0 * 6 + f) * FMAT_STRIDE;
+            riemann_axis<A, TC>(s, vm, Sm, vp, Sp, Mm[MAT_ZP], Mm[MAT_ZS], F[FMAT_ZP],
+                                F[FMAT_ZS], F[FMAT_IZP], F[FMAT_IZS], dv, dT);
+          }
+          TC *o = sfl + f * FC * Nfp + fn_u;
+          if constexpr (FL)
+          {
+            TC L[FACE_LIFT_N];
+            const TC lf = ((EP)geo_tab<TC>(sd) + (size_t)tk.e0 * GEO_STRIDE)[GEO_LX + A];
+            face_lift_axis<A, TC>(s, lf, Mm[MAT_RHOI], Mm[MAT_LAM], Mm[MAT_MU], dv, dT, L);
+#pragma unroll
+            for (int c = 0; c < FACE_LIFT_N; ++c)
+              o[c * Nfp] = L[c];
+          }
+          else
+          {
+#pragma unroll
+            for (int c = 0; c < 3; ++c)
+            {
+              o[c * Nfp] = dv[c];
+              o[(3 + c) * Nfp] = dT[c];
+            }
+          }
+        };
+        if (f < 2)
+          unit(std::integral_constant<int, 0>{});
+        else if (f < 4)
+          unit(std::integral_constant<int, 1>{});
+        else
+          unit(std::integral_constant<int, 2>{});
+      }
+    }
+    __syncthreads();
+  }
+  else if constexpr (PART != PART_VOLUME)
   {
     gptr<const int32_t> nbe = glob(sd.nbr_elem);
     gptr<const uint8_t> nbc = glob(sd.nbr_code);
     gptr<const TC> mtab = mat_tab<TC>(sd);
-    /* tasks axis-major (axis, element, side, face node), so that the
-     * waves of a block mostly see faces of one axis: the flux and lift of
-     * an axis run once per wave, not once per axis present in it */
-    constexpr int TPA = EPB * 2 * Nfp;
 #pragma unroll
     for (int r = 0; r < TPT; ++r)
     {
@@ -259,8 +447,18 @@ __device__ __forceinline__ void elastic_task(const SD &sd, const Task &tk,
         const int et = tk.e0 + lt;
         const int a = fn % n1, b = fn / n1;
         const int nm = face_node<3>(f, n1, a, b);
-        const int32_t ep = nbe[(size_t)et * 6 + f];
-        const int code = nbc[(size_t)et * 6 + f];
+        int32_t ep;
+        int code;
+        if constexpr (EARLY)
+        {
+          ep = fep[r];
+          code = fcode[r];
+        }
+        else
+        {
+          ep = nbe[(size_t)et * 6 + f];
+          code = nbc[(size_t)et * 6 + f];
+        }
         TC *o = sfl + (lt * 6 + f) * FC * Nfp + fn;
         EP Mm = (EP)mtab + (size_t)et * MAT_STRIDE;
         const TC lf = (EP(geo_tab<TC>(sd)) + (size_t)et * GEO_STRIDE)[GEO_LX + A];
@@ -605,7 +803,11 @@ __device__ __forceinline__ void elastic_task(const SD &sd, const Task &tk,
  * 2.88 ms per 48^3 stage).  Multi-element blocks are left to the
  * compiler: capping the four-element FP32 blocks of N = 4 for a third block
  * per CU measured slower (0.594 -> 0.659), as did 8 for FP32 at N = 6 (five
- * blocks per CU, 0.432 -> 0.539). */
+ * blocks per CU, 0.432 -> 0.539).  A block of N = 6 has six wavefronts, two on
+ * half of a CU's SIMDs, and four of them share a CU only where seven
+ * wavefronts fit a SIMD: the FP32 kernel must take at most 72 vector and 96
+ * scalar registers (us per stage at 72 and 94 / 70 and 104 / 74 and 78
+ * registers: 18^3 63 / 73 / 73, resident grid 58 / 77 / 77). */
 template <int N, int EPB, class P> struct NodeWaves
 {
   static constexpr int value =
@@ -670,10 +872,24 @@ template <int N, int EPB, class P> struct NodeSplit
           : 1;
 };
 
+/* blocks per XCD and cube in the block order of the fused kernel (mode 2 of
+ * first_task): 4 x 4 x 4 tasks.  A cube's inner faces are gathered from the
+ * XCD's L2, its outer ones miss it by whole lines (an x face of N = 3 or 7
+ * touches every line of its rows), and a quarter of the faces of a 4 x 4 x 4
+ * cube are outer ones, against half with 2 x 2 x 2.  Read misses per stage,
+ * FP32, in 128-byte lines: N = 3 (30^3) 1.75 M -> 1.34 M, N = 4 (27^3)
+ * 2.49 -> 1.96, N = 6 (18^3) 1.79 -> 1.43, N = 7 (32^3) 13.7 -> 11.2 M.  us per
+ * stage: FP32 N = 3 (30^3) 54.7 -> 52.4, N = 4 (27^3) 82.1 -> 78.5, N = 5
+ * (21^3) 58.6 -> 58.6, N = 6 (18^3) 63.9 -> 64.0, N = 7 (48^3) 1284 -> 1272;
+ * FP64 N = 3 (24^3) 53.2 -> 50.7, N = 4 (20^3) 68.8 -> 66.4; FP32 rates N = 3
+ * (24^3) 47.3 -> 42.0.  512 tasks per cube measured no better at any order
+ * (their window no longer fits an L2 of 4 MB). */
+constexpr int NODE_XC = 64;
+
 /* SPLIT: the launch of a NodeSplit order with NS blocks per task, block v
  * taking elements EPB (v % NS) .. EPB (v % NS) + EPB - 1 of task v / NS */
 template <int N, int EPB, class P, bool SPLIT = false>
-__global__ __launch_bounds__(EPB *(N + 1) * (N + 1) * (N + 1))
+__global__ __launch_bounds__((NodeBlock<N, EPB, P>::value))
 __attribute__((amdgpu_waves_per_eu(NodeWaves<N, EPB, P>::value))) void
 elastic_stage_kernel(LaunchArgs a)
 {
@@ -681,13 +897,15 @@ elastic_stage_kernel(LaunchArgs a)
   /* elements of a node task */
   constexpr int TE = 512 / ((N + 1) * (N + 1) * (N + 1)) < 1 ? 1 : 512 / ((N + 1) * (N + 1) * (N + 1));
   static_assert(TE % EPB == 0, "a block takes whole passes of a task");
-  int stride, end;
   if constexpr (SPLIT)
   {
     constexpr int NS = NodeSplit<N, EPB, P>::value;
     static_assert(NS > 1 && NS * EPB == TE, "split launches take EPB elements per block");
-    for (int vi = first_task(a, a.ntasks * NS, &stride, &end); vi < end; vi += stride)
+    const int n = a.ntasks * NS;
+    const TaskWalk w = task_walk(a, n);
+    for (int v = w.first; v < w.end; v += w.stride)
     {
+      const int vi = task_at<NODE_XC>(a, n, v);
       const int ti = vi / NS, s0 = (vi - ti * NS) * EPB;
       Task tk = load_task(a.tasks, ti);
       if (s0 < tk.ne)
@@ -696,15 +914,16 @@ elastic_stage_kernel(LaunchArgs a)
         const StageCtx cx = stage_ctx(sd, a);
         tk.e0 += s0;
         tk.ne = tk.ne - s0 < EPB ? tk.ne - s0 : EPB;
-        elastic_task<N, EPB, P>(sd, tk, cx, a, smem);
+        elastic_task<N, EPB, P, PART_FUSED, true>(sd, tk, cx, a, smem);
         __syncthreads();
       }
     }
     return;
   }
-  for (int ti = first_task(a, &stride, &end); ti < end; ti += stride)
+  const TaskWalk w = task_walk(a, a.ntasks);
+  for (int v = w.first; v < w.end; v += w.stride)
   {
-    const Task tk = load_task(a.tasks, ti);
+    const Task tk = load_task(a.tasks, task_at<NODE_XC>(a, a.ntasks, v));
     const auto &sd = *(cglob(a.subs) + tk.sub);
     const StageCtx cx = stage_ctx(sd, a);
     if constexpr (EPB == TE)
@@ -730,25 +949,27 @@ template <int N, int EPB, class P>
 static hipError_t launch_ne(const LaunchArgs &a, int grid, hipStream_t s, unsigned dyn)
 {
   constexpr int NS = NodeSplit<N, EPB, P>::value;
-  /* one block per task (not a resident grid): one block per element */
+  /* EPB elements per block, or, on a resident grid (fewer blocks than
+   * tasks), per turn of a block */
   if constexpr (NS > 1)
-    if (grid >= a.ntasks && !a.whole_tasks)
+    if (!a.whole_tasks)
     {
       const int vt = a.ntasks * NS;
-      grid = a.xcd_remap == 1 && a.nxcd > 1 ? a.nxcd * ((vt + a.nxcd - 1) / a.nxcd) : vt;
+      if (grid >= a.ntasks)
+        grid = a.xcd_remap == 1 && a.nxcd > 1 ? a.nxcd * ((vt + a.nxcd - 1) / a.nxcd) : vt;
       hipLaunchKernelGGL((elastic_stage_kernel<N, EPB, P, true>), dim3(grid),
-                         dim3(EPB * (N + 1) * (N + 1) * (N + 1)), dyn, s, a);
+                         dim3(NodeBlock<N, EPB, P>::value), dyn, s, a);
       return hipGetLastError();
     }
   hipLaunchKernelGGL((elastic_stage_kernel<N, EPB, P>), dim3(grid),
-                     dim3(EPB * (N + 1) * (N + 1) * (N + 1)), dyn, s, a);
+                     dim3(NodeBlock<N, EPB, P>::value), dyn, s, a);
   return hipGetLastError();
 }
 template <int N, int EPB, class P>
 static hipError_t occupancy_ne(int *blocks, unsigned dyn)
 {
   return hipOccupancyMaxActiveBlocksPerMultiprocessor(
-      blocks, elastic_stage_kernel<N, EPB, P>, EPB * (N + 1) * (N + 1) * (N + 1), dyn);
+      blocks, elastic_stage_kernel<N, EPB, P>, NodeBlock<N, EPB, P>::value, dyn);
 }
 
 /* alt: the block size of NodeEpbAlt instead of NodeEpb */
@@ -817,14 +1038,14 @@ hipError_t launch_elastic_stage(int prec, int N, const LaunchArgs &a, int grid,
 /* unfused FP64 form: the same element bodies run as a volume kernel and a
  * surface kernel, each a separate pass over HBM through the rhs array */
 template <int N, int EPB, int PART>
-__global__ __launch_bounds__(EPB *(N + 1) * (N + 1) * (N + 1)) void
+__global__ __launch_bounds__((NodeBlock<N, EPB, P64>::value)) void
 elastic_part_kernel(LaunchArgs a)
 {
   __shared__ __align__(16) char smem[NodeLds<N, EPB, P64>::bytes];
-  int stride, end;
-  for (int ti = first_task(a, &stride, &end); ti < end; ti += stride)
+  const TaskWalk w = task_walk(a, a.ntasks);
+  for (int v = w.first; v < w.end; v += w.stride)
   {
-    const Task tk = load_task(a.tasks, ti);
+    const Task tk = load_task(a.tasks, task_at(a, a.ntasks, v));
     const auto &sd = *(cglob(a.subs) + tk.sub);
     const StageCtx cx = stage_ctx(sd, a);
     elastic_task<N, EPB, P64, PART>(sd, tk, cx, a, smem);
@@ -840,10 +1061,9 @@ hipError_t launch_elastic_plain(int N, const LaunchArgs &a, int grid,
 #define BFAMX_CASE(NN, EE)                                                     \
   case NN:                                                                     \
     hipLaunchKernelGGL((elastic_part_kernel<NN, EE, PART_VOLUME>), dim3(grid), \
-                       dim3(EE * (NN + 1) * (NN + 1) * (NN + 1)), 0, s, a);    \
+                       dim3(NodeBlock<NN, EE, P64>::value), 0, s, a);          \
     hipLaunchKernelGGL((elastic_part_kernel<NN, EE, PART_SURFACE>),            \
-                       dim3(grid), dim3(EE * (NN + 1) * (NN + 1) * (NN + 1)),  \
-                       0, s, a);                                               \
+                       dim3(grid), dim3(NodeBlock<NN, EE, P64>::value), 0, s, a);                                               \
     break;
     BFAMX_CASE(3, 8)
     BFAMX_CASE(4, 4)
