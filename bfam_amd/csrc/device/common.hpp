@@ -295,9 +295,6 @@ struct LaunchArgs
   int mode;
   int xcd_remap;
   int nxcd;
-  /* node-parallel stage: one block per task even where the one-element
-   * kernel takes one element per block (an order launched beside others) */
-  int whole_tasks;
   /* stages launched since the clocks were last advanced: the stage's entry
    * of Clock::ctx */
   int slot;

@@ -76,6 +76,10 @@ struct FieldCopy
   }
 };
 
+/* streams that the orders of a batch are dealt to (batch_chains): the
+ * hardware queues of a process */
+constexpr int BATCH_CHAINS = 4;
+
 struct bfamx_device
 {
   int hip_dev;
@@ -114,10 +118,10 @@ struct bfamx_device
    * ~0u unknown) */
   signed char occ[NPREC][9][3];
   unsigned occ_dyn[NPREC][9][3][3];
-  /* the per-order launches of a grouped batch run on side streams forked
-   * from and joined back to `stream` (parallel branches when captured) */
-  hipStream_t side[8];
-  hipEvent_t fork_ev, join_ev[8];
+  /* chains of a grouped batch beside `stream`, forked from and joined back
+   * to it (parallel branches when captured) */
+  hipStream_t side[BATCH_CHAINS - 1];
+  hipEvent_t fork_ev, join_ev[BATCH_CHAINS - 1];
   /* device address of this GPU's copy of `scratch` (bfamx_rhs_noalloc) */
   double *scratch;
   FieldCopy fc;
@@ -276,7 +280,7 @@ extern "C" int bfamx_device_create(int hip_device, size_t hbm_budget_bytes,
   HIPCHK(hipEventCreate(&d->ev0));
   HIPCHK(hipEventCreate(&d->ev1));
   HIPCHK(hipEventCreateWithFlags(&d->fork_ev, hipEventDisableTiming));
-  for (int i = 0; i < 8; ++i)
+  for (int i = 0; i < BATCH_CHAINS - 1; ++i)
   {
     HIPCHK(hipStreamCreateWithFlags(&d->side[i], hipStreamNonBlocking));
     HIPCHK(hipEventCreateWithFlags(&d->join_ev[i], hipEventDisableTiming));
@@ -294,7 +298,7 @@ extern "C" int bfamx_device_destroy(bfamx_device_t *d)
   (void)hipEventDestroy(d->ev0);
   (void)hipEventDestroy(d->ev1);
   (void)hipEventDestroy(d->fork_ev);
-  for (int i = 0; i < 8; ++i)
+  for (int i = 0; i < BATCH_CHAINS - 1; ++i)
   {
     (void)hipStreamSynchronize(d->side[i]);
     (void)hipStreamDestroy(d->side[i]);
@@ -1799,21 +1803,6 @@ static GlueArgs glue_args(const bfamx_batch_t *b)
   return g;
 }
 
-/* the order of a batch with the most volume nodes (the one launched on the
- * batch's stream when orders launch side by side) */
-static int batch_big_order(const bfamx_batch_t *b)
-{
-  int big = -1;
-  for (int n = 0; n < 9; ++n)
-    if (b->grp_cnt[n] &&
-        (big < 0 || (size_t)b->grp_cnt[n] * (n + 1) * (n + 1) * (n + 1) >
-                        (size_t)b->grp_cnt[big] * (big + 1) * (big + 1) * (big + 1)))
-      big = n;
-  return big;
-}
-
-/* the stage kernels of a batch: one launch (one order, or all orders with
- * the mixed kernel), or one launch per order over its slice of the tasks */
 /* the stage kernels of the orders [n] of a batch with their chosen kernel:
  * the line kernel over the line tasks, or the node-parallel kernel over the
  * node tasks */
@@ -1825,9 +1814,6 @@ static hipError_t launch_order(bfamx_batch_t *b, const LaunchArgs &a, int n,
   {
     g.tasks = b->d_tasks_node + b->grpn_off[n];
     g.ntasks = b->grpn_cnt[n];
-    /* an order that runs beside the batch's largest keeps whole tasks,
-     * in the autotuner's trials as in the batch stage */
-    g.whole_tasks = b->N < 0 && n != batch_big_order(b);
     const int slot = kernel_slot(b->dev, b->prec, n);
     return launch_elastic_stage(b->prec, n, g, grid_node(b->dev, b->prec, n, g.ntasks), st,
                                 kernel_dyn(b->dev, b->prec, n, slot), slot == 2);
@@ -1842,11 +1828,78 @@ static hipError_t launch_order(bfamx_batch_t *b, const LaunchArgs &a, int n)
   return launch_order(b, a, n, b->dev->stream);
 }
 
+/* The streams of a batch's order launches: order n on chain at[n], 0 the
+ * batch's stream.  The orders of a batch without mortars never read each
+ * other's states, so up to BATCH_CHAINS chains of stages run side by side
+ * and meet only where the clocks advance: one chain's small launches fill
+ * the last waves of another's.  Orders go to the chain with the least volume
+ * nodes, largest first.  Six members of orders 3..7 (0.2-0.9 M values a
+ * member and field, FP32), us per stage: a fork and a join around every stage
+ * 93; one stream 81; chains over ten steps 68 (two), 67 (three), 62 (four);
+ * five on the four hardware queues 63.  Mortars read all orders between two
+ * stages: one stream then (adapted mesh, orders 7/5/3: 102, with a fork and a
+ * join per stage 102). */
+struct BatchChains
+{
+  int n, at[9];
+};
+static BatchChains batch_chains(const bfamx_batch_t *b)
+{
+  BatchChains c;
+  memset(&c, 0, sizeof(c));
+  c.n = 1;
+  if (b->glue || !b->grouped)
+    return c;
+  size_t nodes[9] = {0}, load[BATCH_CHAINS] = {0};
+  for (auto *s : b->subs)
+    nodes[s->N] += (size_t)s->K * s->Np;
+  for (;;)
+  {
+    int big = 0;
+    for (int n = 1; n < 9; ++n)
+      if (nodes[n] > nodes[big])
+        big = n;
+    if (nodes[big] == 0)
+      return c;
+    int k = 0;
+    for (int i = 1; i < BATCH_CHAINS; ++i)
+      if (load[i] < load[k])
+        k = i;
+    c.at[big] = k;
+    load[k] += nodes[big];
+    nodes[big] = 0;
+    c.n = k + 1 > c.n ? k + 1 : c.n;
+  }
+}
+static hipError_t fork_chains(const bfamx_batch_t *b, const BatchChains &ch)
+{
+  bfamx_device_t *d = b->dev;
+  hipError_t e = ch.n > 1 ? hipEventRecord(d->fork_ev, d->stream) : hipSuccess;
+  for (int k = 0; k < ch.n - 1 && e == hipSuccess; ++k)
+    e = hipStreamWaitEvent(d->side[k], d->fork_ev, 0);
+  return e;
+}
+/* every chain is joined, also after a failed one */
+static hipError_t join_chains(const bfamx_batch_t *b, const BatchChains &ch)
+{
+  bfamx_device_t *d = b->dev;
+  hipError_t first = hipSuccess;
+  for (int k = 0; k < ch.n - 1; ++k)
+  {
+    hipError_t e = hipEventRecord(d->join_ev[k], d->side[k]);
+    if (e == hipSuccess)
+      e = hipStreamWaitEvent(d->stream, d->join_ev[k], 0);
+    if (first == hipSuccess)
+      first = e;
+  }
+  return first;
+}
+
 /* the stage kernels of a batch: one launch (one order, or all orders with
  * the order-switching kernel), or one launch per order over its slice of
  * the tasks */
 static hipError_t launch_batch_kernels(bfamx_batch_t *b, const LaunchArgs &a,
-                                       int grid)
+                                       int grid, const BatchChains &ch)
 {
   if (b->physics != BFAMX_ELASTIC3D)
     return launch_acoustic_stage(b->prec, b->N, a, grid, b->dev->stream);
@@ -1855,39 +1908,16 @@ static hipError_t launch_batch_kernels(bfamx_batch_t *b, const LaunchArgs &a,
   if (!b->grouped)
     return launch_elastic_line(b->prec, b->N, a, grid_line(b->dev, b->prec, b->N, a.ntasks),
                                b->dev->stream);
-  /* one launch per order: the largest on the batch's stream, the others on
-   * side streams forked after and joined before the next launch, so small
-   * orders do not wait for the tail of a large one */
-  int ord[9], no = 0;
-  const int big = batch_big_order(b);
-  for (int n = 0; n < 9; ++n)
-    if (b->grp_cnt[n])
-      ord[no++] = n;
-  bfamx_device_t *d = b->dev;
+  /* one launch per order, on the stream of its chain */
   hipError_t e = hipSuccess;
-  if (no > 1)
-    e = hipEventRecord(d->fork_ev, d->stream);
-  int k = 0;
-  for (int i = 0; i < no && e == hipSuccess; ++i)
-  {
-    if (ord[i] == big)
-      continue;
-    e = hipStreamWaitEvent(d->side[k], d->fork_ev, 0);
-    if (e == hipSuccess)
-      e = launch_order(b, a, ord[i], d->side[k]);
-    if (e == hipSuccess)
-      e = hipEventRecord(d->join_ev[k], d->side[k]);
-    ++k;
-  }
-  if (e == hipSuccess && big >= 0)
-    e = launch_order(b, a, big, d->stream);
-  for (int i = 0; i < k && e == hipSuccess; ++i)
-    e = hipStreamWaitEvent(d->stream, d->join_ev[i], 0);
+  for (int n = 0; n < 9 && e == hipSuccess; ++n)
+    if (b->grp_cnt[n])
+      e = launch_order(b, a, n, ch.at[n] ? b->dev->side[ch.at[n] - 1] : b->dev->stream);
   return e;
 }
 
 /* the kernels of the stage whose parameters are in `slot` of the clocks */
-static int batch_stage(bfamx_batch_t *b, int slot)
+static int batch_stage(bfamx_batch_t *b, int slot, const BatchChains &ch)
 {
   LaunchArgs a;
   memset(&a, 0, sizeof(a));
@@ -1907,7 +1937,7 @@ static int batch_stage(bfamx_batch_t *b, int slot)
     e = launch_mortar(b->prec, g, b->dev->stream);
   }
   if (e == hipSuccess)
-    e = launch_batch_kernels(b, a, grid);
+    e = launch_batch_kernels(b, a, grid, ch);
   if (e != hipSuccess)
     return bfamx_fail(BFAMX_EHIP, "batch stage launch: %s", hipGetErrorString(e));
   return BFAMX_OK;
@@ -1918,15 +1948,21 @@ static int batch_stage(bfamx_batch_t *b, int slot)
 static int batch_run(bfamx_batch_t *b, long long n, long long *done)
 {
   int rc = BFAMX_OK;
+  const BatchChains ch = batch_chains(b);
   *done = 0;
   while (n > 0 && !rc)
   {
     const int m = n < CLOCK_SLOTS ? (int)n : CLOCK_SLOTS;
     int k = 0;
-    while (k < m && !(rc = batch_stage(b, k)))
+    hipError_t e = fork_chains(b, ch);
+    if (e != hipSuccess)
+      rc = bfamx_fail(BFAMX_EHIP, "batch fork: %s", hipGetErrorString(e));
+    while (k < m && !rc && !(rc = batch_stage(b, k, ch)))
       ++k;
-    const hipError_t e =
-        launch_clock_advance(b->d_subs, (int)b->subs.size(), k, 0, b->dev->stream);
+    e = join_chains(b, ch);
+    if (e != hipSuccess && !rc)
+      rc = bfamx_fail(BFAMX_EHIP, "batch join: %s", hipGetErrorString(e));
+    e = launch_clock_advance(b->d_subs, (int)b->subs.size(), k, 0, b->dev->stream);
     if (e != hipSuccess && !rc)
       rc = bfamx_fail(BFAMX_EHIP, "clock launch failed: %s", hipGetErrorString(e));
     *done += k;
@@ -2547,8 +2583,16 @@ extern "C" int bfamx_batch_autotune(bfamx_batch_t *b, int trials, int force,
     for (int mode = 0; mode < 2 && !rc; ++mode)
     {
       b->grouped = mode;
-      rc = time_it([&]() { return launch_batch_kernels(b, a, grid_for(d, b->ntasks)); },
-                   &ms[mode]);
+      rc = time_it(
+          [&]() {
+            const BatchChains ch = batch_chains(b);
+            hipError_t e = fork_chains(b, ch);
+            if (e == hipSuccess)
+              e = launch_batch_kernels(b, a, grid_for(d, b->ntasks), ch);
+            const hipError_t ej = join_chains(b, ch);
+            return e == hipSuccess ? ej : e;
+          },
+          &ms[mode]);
     }
     if (!rc)
       mc = (signed char)(ms[1] < ms[0] ? 1 : 0);
