@@ -298,9 +298,27 @@ struct LaunchArgs
   /* stages launched since the clocks were last advanced: the stage's entry
    * of Clock::ctx */
   int slot;
+  /* a launch over the whole of one subdomain, its tasks in element order:
+   * the slots of its clock, its descriptor's index and its elements
+   * (launch_task).  NULL: the task table and the descriptors' clocks. */
+  const StageSlot *one;
+  int one_sub, one_K;
   /* MODE_RHS: ricker(t), sin and cos(omega t) at the caller's time */
   double g_rhs, sw_rhs, cw_rhs;
 };
+
+/* Task i of a launch whose tasks hold TE elements.  ONE: computed where the
+ * launch names its subdomain, and the stage parameters then loaded beside the
+ * descriptor (stage_ctx): two dependent scalar loads fewer before a block
+ * requests its state. */
+template <int TE, bool ONE>
+__device__ __forceinline__ Task launch_task(const LaunchArgs &a, int i)
+{
+  if (!ONE || !a.one)
+    return load_task(a.tasks, i);
+  const int e0 = i * TE, left = a.one_K - e0;
+  return {a.one_sub, e0, left < TE ? left : TE, 0};
+}
 
 /* element-major offset of (element, field, node) */
 __device__ __forceinline__ size_t qidx(int e, int f, int n, int NF, int Np)
@@ -366,11 +384,12 @@ struct StageCtx
 /* SD: SubDev, possibly qualified with the constant address space.  The
  * clock is constant within a stage launch: only clock_advance_kernel, a
  * separate launch, writes it. */
-template <class SD>
+template <bool ONE = false, class SD>
 __device__ __forceinline__ StageCtx stage_ctx(const SD &sd, const LaunchArgs &a)
 {
   StageCtx c;
-  c.slot = cglob((const StageSlot *)((const Clock *)sd.clock)->ctx) + a.slot;
+  const StageSlot *own = ((const Clock *)sd.clock)->ctx;
+  c.slot = cglob(ONE && a.one ? a.one : own) + a.slot;
   const bool stage = a.mode != MODE_RHS;
   c.parity = c.slot->parity;
   c.dq_dead = stage ? c.slot->dq_dead : 0;

@@ -1167,6 +1167,8 @@ static LaunchArgs launch_args(bfamx_subdomain_t *s, int mode)
   a.mode = mode;
   a.xcd_remap = s->dev->xcd_remap;
   a.nxcd = s->dev->num_xcd;
+  a.one = s->d_clock->ctx;
+  a.one_K = s->K;
   return a;
 }
 
@@ -1803,6 +1805,24 @@ static GlueArgs glue_args(const bfamx_batch_t *b)
   return g;
 }
 
+/* a launch over the subdomains of order n names the subdomain if it is the
+ * only one (LaunchArgs::one) */
+static void only_sub(const bfamx_batch_t *b, int n, LaunchArgs *a)
+{
+  int at = -1, count = 0;
+  for (size_t i = 0; i < b->subs.size(); ++i)
+    if (b->subs[i]->N == n)
+    {
+      at = (int)i;
+      ++count;
+    }
+  if (count != 1)
+    return;
+  a->one = b->subs[at]->d_clock->ctx;
+  a->one_sub = at;
+  a->one_K = b->subs[at]->K;
+}
+
 /* the stage kernels of the orders [n] of a batch with their chosen kernel:
  * the line kernel over the line tasks, or the node-parallel kernel over the
  * node tasks */
@@ -1810,6 +1830,7 @@ static hipError_t launch_order(bfamx_batch_t *b, const LaunchArgs &a, int n,
                                hipStream_t st)
 {
   LaunchArgs g = a;
+  only_sub(b, n, &g);
   if (node_kernel(b->dev, b->prec, n))
   {
     g.tasks = b->d_tasks_node + b->grpn_off[n];

@@ -882,6 +882,20 @@ template <int N, int EPB, class P> struct NodeSplit
  * (their window no longer fits an L2 of 4 MB). */
 constexpr int NODE_XC = 64;
 
+/* whether the stage kernel computes its task where the launch names its one
+ * subdomain (LaunchArgs::one) or loads it from the table.  us per stage,
+ * loaded / computed: N = 7 FP32 1227 / 1208 (48^3), 364 / 358 (32^3), FP64 391 /
+ * 387 (26^3), FP32 rates 1232 / 1227 (40^3); FP64 N = 4 62.5 / 61.3 (20^3), N = 6
+ * 323 / 320 (26^3); FP32 rates N = 6 400 / 387 (28^3).  Elsewhere the registers
+ * that the choice takes cost more: FP32 N = 6 57.7 / 76.4 (18^3), FP32 rates
+ * N = 4 55.1 / 58.6 (20^3), FP64 N = 5 69.7 / 71.7 (18^3), or it is the same (FP32
+ * N = 3, 4). */
+template <int N, class P> struct NodeOne
+{
+  static constexpr bool value = N == 7 || (__is_same(P, P64) && N != 5) ||
+                                (__is_same(P, P32R) && N == 6);
+};
+
 /* SPLIT: the launch of a NodeSplit order with NS blocks per task, block v
  * taking elements EPB (v % NS) .. EPB (v % NS) + EPB - 1 of task v / NS */
 template <int N, int EPB, class P, bool SPLIT = false>
@@ -903,11 +917,11 @@ elastic_stage_kernel(LaunchArgs a)
     {
       const int vi = task_at<NODE_XC>(a, n, v);
       const int ti = vi / NS, s0 = (vi - ti * NS) * EPB;
-      Task tk = load_task(a.tasks, ti);
+      Task tk = launch_task<TE, NodeOne<N, P>::value>(a, ti);
       if (s0 < tk.ne)
       {
         const auto &sd = *(cglob(a.subs) + tk.sub);
-        const StageCtx cx = stage_ctx(sd, a);
+        const StageCtx cx = stage_ctx<NodeOne<N, P>::value>(sd, a);
         tk.e0 += s0;
         tk.ne = tk.ne - s0 < EPB ? tk.ne - s0 : EPB;
         elastic_task<N, EPB, P, PART_FUSED, true>(sd, tk, cx, a, smem);
@@ -919,9 +933,9 @@ elastic_stage_kernel(LaunchArgs a)
   const TaskWalk w = task_walk(a, a.ntasks);
   for (int v = w.first; v < w.end; v += w.stride)
   {
-    const Task tk = load_task(a.tasks, task_at<NODE_XC>(a, a.ntasks, v));
+    const Task tk = launch_task<TE, NodeOne<N, P>::value>(a, task_at<NODE_XC>(a, a.ntasks, v));
     const auto &sd = *(cglob(a.subs) + tk.sub);
-    const StageCtx cx = stage_ctx(sd, a);
+    const StageCtx cx = stage_ctx<NodeOne<N, P>::value>(sd, a);
     if constexpr (EPB == TE)
     {
       elastic_task<N, EPB, P>(sd, tk, cx, a, smem);
