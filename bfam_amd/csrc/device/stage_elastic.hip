@@ -34,6 +34,7 @@
  * The task, descriptor, clock and, for one-element blocks, the element
  * tables are read through the constant address space (scalar loads).
  */
+#include <climits>
 #include <type_traits>
 
 #include "elastic_axis.hpp"
@@ -70,11 +71,15 @@ template <int N> struct NodeFaceLift
  * stage, tasks / units: N = 7 FP32 1272 / 1250 (48^3), 378 / 372 (32^3), 51.5 /
  * 50.5 (16^3); FP64 1534 / 1420 (40^3, resident grid); FP32 rates 1350 / 1236
  * (40^3), 95 / 86 (16^3), where FP64 traces are six loads of two registers;
- * N = 6 FP32 rates 420 / 391 (28^3), 96 / 91 (17^3). */
+ * N = 6 FP32 rates 420 / 391 (28^3), 96 / 91 (17^3); N = 5 (36 of 64 lanes,
+ * six units on four wavefronts, one block per element) FP64 340 / 306 (32^3),
+ * 67.3 / 60.6 (18^3), FP32 297 / 292 (38^3), 54.8 / 53.9 (21^3), but FP32 rates
+ * 59.7 / 63.2 (18^3). */
 template <int N, int EPB, class P> struct NodeUnits
 {
+  static constexpr bool rates32 = __is_same(P, P32R);
   static constexpr bool value =
-      EPB == 1 && !P::MF && (N == 7 || (N == 6 && __is_same(P, P32R)));
+      EPB == 1 && !P::MF && (N == 7 || (N == 6 && rates32) || (N == 5 && !rates32));
 };
 
 /* threads of a block: its volume nodes, and for face units whole wavefronts */
@@ -853,19 +858,20 @@ template <int N, class P> struct NodeEpbAlt
  * one block taking the whole task in passes, 1 elsewhere.  FP64 at N = 3
  * (two-element blocks): 0.805 -> 0.789 ms per stage.  Each XCD's
  * blocks then cover 2x2x2 elements of a Morton group instead of 4x4x4
- * (N = 3), and fewer elements are in flight per XCD.  ms per stage on
- * bricks of about 124 M DOF: FP32 N = 3 0.443 -> 0.412-0.414, N = 4
- * 0.548-0.552 -> 0.523-0.530.  FP32 at N = 5 measured slower with
- * one-element tasks (0.455 -> 0.464), as did the resident grids; the FP64
- * N = 4 form spilled 12 bytes per lane and took 0.866 -> 0.946 ms. */
+ * (N = 3), and fewer elements are in flight per XCD, and a small subdomain
+ * spreads over as many CUs as it has elements.  ms per stage on bricks of
+ * about 124 M DOF: FP32 N = 3 0.443 -> 0.412-0.414, N = 4 0.548-0.552 ->
+ * 0.523-0.530.  us per stage, whole tasks / split: N = 5 FP32 316 / 297 (38^3),
+ * 58.9 / 54.8 (21^3), 12.4 / 10.2 (10^3), 10.4 / 7.3 (6^3), FP32 rates 260 / 257
+ * (30^3), 64.2 / 59.6 (18^3), 12.8 / 8.7 (8^3), FP64 364 / 340 (32^3), 69.6 / 67.3
+ * (18^3), 12.9 / 9.3 (8^3); FP64 N = 4 (12 bytes of spill per lane) 23.3 /
+ * 7.7 (4^3), 61.6 / 59.8 (20^3), 164 / 156 (28^3), but 290 / 304 (34^3): whole
+ * tasks from max_tasks on. */
 template <int N, int EPB, class P> struct NodeSplit
 {
   static constexpr int TE = 512 / ((N + 1) * (N + 1) * (N + 1)) < 1 ? 1 : 512 / ((N + 1) * (N + 1) * (N + 1));
-  static constexpr int value =
-      (EPB == 1 && (__is_same(P, P32) || __is_same(P, P32R)) && (N == 3 || N == 4)) ||
-              (EPB == 2 && __is_same(P, P64) && N == 3)
-          ? TE / EPB
-          : 1;
+  static constexpr int value = !P::MF && EPB == NodeEpb<N, P>::value ? TE / EPB : 1;
+  static constexpr int max_tasks = N == 4 && __is_same(P, P64) ? 7168 : INT_MAX;
 };
 
 /* blocks per XCD and cube in the block order of the fused kernel (mode 2 of
@@ -888,12 +894,12 @@ constexpr int NODE_XC = 64;
  * 387 (26^3), FP32 rates 1232 / 1227 (40^3); FP64 N = 4 62.5 / 61.3 (20^3), N = 6
  * 323 / 320 (26^3); FP32 rates N = 6 400 / 387 (28^3).  Elsewhere the registers
  * that the choice takes cost more: FP32 N = 6 57.7 / 76.4 (18^3), FP32 rates
- * N = 4 55.1 / 58.6 (20^3), FP64 N = 5 69.7 / 71.7 (18^3), or it is the same (FP32
- * N = 3, 4). */
+ * N = 4 55.1 / 58.6 (20^3), N = 5 285 / 307 (30^3), or it is the same (FP32 N = 3,
+ * 4).  N = 5: FP32 301 / 292 (38^3), FP64 312 / 306 (32^3). */
 template <int N, class P> struct NodeOne
 {
-  static constexpr bool value = N == 7 || (__is_same(P, P64) && N != 5) ||
-                                (__is_same(P, P32R) && N == 6);
+  static constexpr bool value = N == 7 || __is_same(P, P64) || (__is_same(P, P32R) && N == 6) ||
+                                (__is_same(P, P32) && N == 5);
 };
 
 /* SPLIT: the launch of a NodeSplit order with NS blocks per task, block v
@@ -963,14 +969,15 @@ static hipError_t launch_ne(const LaunchArgs &a, int grid, hipStream_t s, unsign
   /* EPB elements per block, or, on a resident grid (fewer blocks than
    * tasks), per turn of a block */
   if constexpr (NS > 1)
-  {
-    const int vt = a.ntasks * NS;
-    if (grid >= a.ntasks)
-      grid = a.xcd_remap == 1 && a.nxcd > 1 ? a.nxcd * ((vt + a.nxcd - 1) / a.nxcd) : vt;
-    hipLaunchKernelGGL((elastic_stage_kernel<N, EPB, P, true>), dim3(grid),
-                       dim3(NodeBlock<N, EPB, P>::value), dyn, s, a);
-    return hipGetLastError();
-  }
+    if (a.ntasks < NodeSplit<N, EPB, P>::max_tasks)
+    {
+      const int vt = a.ntasks * NS;
+      if (grid >= a.ntasks)
+        grid = a.xcd_remap == 1 && a.nxcd > 1 ? a.nxcd * ((vt + a.nxcd - 1) / a.nxcd) : vt;
+      hipLaunchKernelGGL((elastic_stage_kernel<N, EPB, P, true>), dim3(grid),
+                         dim3(NodeBlock<N, EPB, P>::value), dyn, s, a);
+      return hipGetLastError();
+    }
   hipLaunchKernelGGL((elastic_stage_kernel<N, EPB, P>), dim3(grid),
                      dim3(NodeBlock<N, EPB, P>::value), dyn, s, a);
   return hipGetLastError();
