@@ -715,6 +715,20 @@ __device__ __forceinline__ void elastic_task(const SD &sd, const Task &tk,
     BFAMX_LIFT(2, k, i + n1 * j)
 #undef BFAMX_LIFT
   }
+  else if constexpr (PART != PART_VOLUME && N == 3 && __is_same(P, P32))
+  {
+    /* one wavefront meets all six faces: one branch per axis, for the face
+     * of the axis the node lies on, runs three lifts instead of six.  us per
+     * stage, six branches / three: 50.2 / 49.2 (30^3), 289 / 284 (56^3), 6.17 /
+     * 6.05 (8^3); FP32 N = 6 then takes over 96 scalar registers (NodeWaves) */
+    const TC *F = sfl + le * 6 * FC * Nfp;
+    TC flv[6];
+#define BFAMX_LIFT(A, c_, fn_)                                                   if ((c_) == 0 || (c_) == N)                                                    {                                                                                const TC *Ff = F + (2 * (A) + ((c_) == N)) * FC * Nfp + (fn_);                 _Pragma("unroll") for (int c = 0; c < 6; ++c) flv[c] = Ff[c * Nfp];            elastic_lift<TC>(A, (c_) == N ? TC(1) : TC(-1), G[GEO_LX + (A)], rhoi,                          lam, mu, flv, rate);                                        }
+    BFAMX_LIFT(0, i, j + n1 * k)
+    BFAMX_LIFT(1, j, i + n1 * k)
+    BFAMX_LIFT(2, k, i + n1 * j)
+#undef BFAMX_LIFT
+  }
   else if constexpr (PART != PART_VOLUME)
   {
     const TC *F = sfl + le * 6 * FC * Nfp;
