@@ -1923,7 +1923,11 @@ static hipError_t launch_batch_kernels(bfamx_batch_t *b, const LaunchArgs &a,
                                        int grid, const BatchChains &ch)
 {
   if (b->physics != BFAMX_ELASTIC3D)
-    return launch_acoustic_stage(b->prec, b->N, a, grid, b->dev->stream);
+  {
+    LaunchArgs g = a;
+    only_sub(b, b->N, &g);
+    return launch_acoustic_stage(b->prec, b->N, g, grid, b->dev->stream);
+  }
   if (b->N >= 0)
     return launch_order(b, a, b->N);
   if (!b->grouped)

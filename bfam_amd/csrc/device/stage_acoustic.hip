@@ -18,8 +18,8 @@ template <int N, int EPB, class T> struct AcousticSmem
   static constexpr int n1 = N + 1, Np = n1 * n1;
   static constexpr int QW = EPB * 3 * Np;
   static constexpr int FW = EPB * 4 * n1;
-  static constexpr int W = QW > FW ? QW : FW;
-  static constexpr size_t bytes = sizeof(T) * (W + n1 * n1);
+  /* LDS: fields, face values, D */
+  static constexpr size_t bytes = sizeof(T) * (QW + FW + n1 * n1);
 };
 
 template <int N, int EPB, class P, int PART = PART_FUSED, class SD>
@@ -42,36 +42,107 @@ __device__ __forceinline__ void acoustic_task(const SD &sd, const Task &tk,
   const int e = tk.e0 + le;
   const int i = n % n1, j = n / n1;
 
-  TC *sq = reinterpret_cast<TC *>(smem);
-  TC *sD = sq + SM::W;
-  {
-    gptr<const TC> Dg = dr_tab<TC>(sd);
-    for (int t = tid; t < n1 * n1; t += blockDim.x)
-      sD[t] = Dg[t];
-  }
+  TC *sq = reinterpret_cast<TC *>(smem); /* [EPB][3][Np] */
+  TC *sfl = sq + SM::QW;                 /* [EPB][4][Nfp] */
+  TC *sD = sfl + SM::FW;
 
+  /* Everything the block reads from memory is requested here, the face traces
+   * once the indices are there, so that a stage takes two round trips after
+   * its descriptor's instead of five: a small subdomain's stage is that chain
+   * of latencies, and a large one's occupancy covers them better.  us per
+   * stage, loads at their use / here: FP64 N = 4 5.01 / 4.28 (16^2), 39.7 / 27.5
+   * (256^2), N = 7 25.4 / 18.1 (128^2), FP32 N = 3 14.8 / 11.9 (256^2) */
   gptr<const TS> qin = glob(static_cast<const TS *>(sd.q[cx.parity]));
+  int32_t ep[TPT];
+  int code[TPT];
+  if constexpr (PART != PART_VOLUME)
+  {
+#pragma unroll
+    for (int r = 0; r < TPT; ++r)
+    {
+      const int t = tid + r * BS;
+      const int lt = t / (4 * Nfp);
+      if (tid < BS && t < NT && lt < tk.ne)
+      {
+        const size_t fi = (size_t)(tk.e0 + lt) * 4 + (t - lt * 4 * Nfp) / Nfp;
+        ep[r] = glob(sd.nbr_elem)[fi];
+        code[r] = glob(sd.nbr_code)[fi];
+      }
+    }
+  }
+  const bool upd = !(la.mode == MODE_RHS || PART != PART_FUSED);
+  /* A = 0 (first stage of a step): no dq read.  FP32, FP64: the old dq is
+   * rebuilt from the previous state, B_{s-1} dq_{s-1} = q_s - q_{s-1}, read
+   * from the other ping-pong buffer before this thread overwrites the node (a
+   * holds A_s / B_{s-1}) */
+  const bool rd_dq = upd && cx.a != 0.0;
+  constexpr bool REC = sizeof(TS) == sizeof(TR);
+  const bool rec = REC && cx.rec;
+  gptr<TS> qout = glob(static_cast<TS *>(sd.q[cx.parity ^ 1]));
+  gptr<TR> dqp = glob(static_cast<TR *>(sd.dq));
   TS qs[NF];
+  TR old[NF];
+  TC rhoi = 0, bulk = 0, Zm = 0, gx = 0, gy = 0, lx = 0, ly = 0;
   if (act)
   {
 #pragma unroll
     for (int f = 0; f < NF; ++f)
-    {
       qs[f] = qin[qidx(e, f, n, NF, Np)];
-      sq[(le * NF + f) * Np + n] = (TC)qs[f];
-    }
-  }
-  __syncthreads();
-
-  TC rate[NF];
-  TC rhoi = 0, bulk = 0, Zm = 0;
-  if (act)
-  {
     gptr<const TC> M = mat_tab<TC>(sd) + (size_t)e * MAT_STRIDE;
     rhoi = M[MAT_RHOI];
     bulk = M[MAT_LAM];
     Zm = M[MAT_ZP];
+    gptr<const TC> G = geo_tab<TC>(sd) + (size_t)e * GEO_STRIDE;
+    gx = G[GEO_GX];
+    gy = G[GEO_GY];
+    lx = G[GEO_LX];
+    ly = G[GEO_LY];
+    if (rd_dq)
+    {
+      gptr<const TR> o = rec ? (gptr<const TR>)qout : (gptr<const TR>)dqp;
+#pragma unroll
+      for (int f = 0; f < NF; ++f)
+        old[f] = o[qidx(e, f, n, NF, Np)];
+    }
   }
+  TC Dv = 0;
+  gptr<const TC> Dg = dr_tab<TC>(sd);
+  if (tid < n1 * n1)
+    Dv = Dg[tid];
+  /* plus trace (p, v_axis) and both impedances of this thread's face nodes */
+  TS gp[TPT], gv[TPT];
+  TC zm[TPT], zp[TPT];
+  if constexpr (PART != PART_VOLUME)
+  {
+#pragma unroll
+    for (int r = 0; r < TPT; ++r)
+    {
+      const int t = tid + r * BS;
+      const int lt = t / (4 * Nfp);
+      if (tid < BS && t < NT && lt < tk.ne)
+      {
+        const int rem = t - lt * 4 * Nfp;
+        const int f = rem / Nfp, a = rem - (rem / Nfp) * Nfp;
+        const int np = nbr_node(code[r], f, n1, face_node<2>(f, n1, a, 0));
+        gp[r] = qin[qidx(ep[r], 0, np, NF, Np)];
+        gv[r] = qin[qidx(ep[r], 1 + (f >> 1), np, NF, Np)];
+        zm[r] = (mat_tab<TC>(sd) + (size_t)(tk.e0 + lt) * MAT_STRIDE)[MAT_ZP];
+        zp[r] = (mat_tab<TC>(sd) + (size_t)ep[r] * MAT_STRIDE)[MAT_ZP];
+      }
+    }
+  }
+  if (tid < n1 * n1)
+    sD[tid] = Dv;
+  static_assert(BS >= n1 * n1, "one D entry per thread");
+  if (act)
+  {
+#pragma unroll
+    for (int f = 0; f < NF; ++f)
+      sq[(le * NF + f) * Np + n] = (TC)qs[f];
+  }
+  __syncthreads();
+
+  TC rate[NF];
   if (act && PART == PART_SURFACE)
   {
 #pragma unroll
@@ -80,7 +151,6 @@ __device__ __forceinline__ void acoustic_task(const SD &sd, const Task &tk,
   }
   if (act && PART != PART_SURFACE)
   {
-    gptr<const TC> G = geo_tab<TC>(sd) + (size_t)e * GEO_STRIDE;
     const TC *u = sq + le * NF * Np;
     TC px = 0, ux = 0, py = 0, vy = 0;
 #pragma unroll
@@ -99,7 +169,6 @@ __device__ __forceinline__ void acoustic_task(const SD &sd, const Task &tk,
       py += c * u[0 * Np + id];
       vy += c * u[2 * Np + id];
     }
-    const TC gx = G[GEO_GX], gy = G[GEO_GY];
     px *= gx, ux *= gx, py *= gy, vy *= gy;
     rate[0] = -bulk * (ux + vy);
     rate[1] = -px * rhoi;
@@ -108,65 +177,46 @@ __device__ __forceinline__ void acoustic_task(const SD &sd, const Task &tk,
 
   if constexpr (PART != PART_VOLUME)
   {
-  TC fl[TPT];
 #pragma unroll
-  for (int r = 0; r < TPT; ++r)
-  {
-    const int t = tid + r * BS;
-    const int lt = t / (4 * Nfp);
-    if (tid < BS && t < NT && lt < tk.ne)
+    for (int r = 0; r < TPT; ++r)
     {
-      const int rem = t - lt * 4 * Nfp;
-      const int f = rem / Nfp, a = rem - (rem / Nfp) * Nfp;
-      const int et = tk.e0 + lt;
-      const int nm = face_node<2>(f, n1, a, 0);
-      const int32_t ep = glob(sd.nbr_elem)[(size_t)et * 4 + f];
-      const int code = glob(sd.nbr_code)[(size_t)et * 4 + f];
-      const int np = nbr_node(code, f, n1, nm);
-      const TC *u = sq + lt * NF * Np;
-      const int axis = f >> 1;
-      const TC s = (f & 1) ? TC(1) : TC(-1);
-      TC sv, ss; /* pressure plays the stress: free surface p+ = -p- */
-      nbr_mirror<TC>(code, &sv, &ss);
-      const TC pm = u[nm], vnm = s * u[(1 + axis) * Np + nm];
-      const TC pp = ss * (TC)qin[qidx(ep, 0, np, NF, Np)];
-      const TC vnp = sv * s * (TC)qin[qidx(ep, 1 + axis, np, NF, Np)];
-      gptr<const TC> Mm = mat_tab<TC>(sd) + (size_t)et * MAT_STRIDE;
-      gptr<const TC> Mp = mat_tab<TC>(sd) + (size_t)ep * MAT_STRIDE;
-      fl[r] = (Mp[MAT_ZP] * (vnp - vnm) + (pm - pp)) / (Mm[MAT_ZP] + Mp[MAT_ZP]);
+      const int t = tid + r * BS;
+      const int lt = t / (4 * Nfp);
+      if (tid < BS && t < NT && lt < tk.ne)
+      {
+        const int rem = t - lt * 4 * Nfp;
+        const int f = rem / Nfp, a = rem - (rem / Nfp) * Nfp;
+        const int nm = face_node<2>(f, n1, a, 0);
+        const TC *u = sq + lt * NF * Np;
+        const TC s = (f & 1) ? TC(1) : TC(-1);
+        TC sv, ss; /* pressure plays the stress: free surface p+ = -p- */
+        nbr_mirror<TC>(code[r], &sv, &ss);
+        const TC pm = u[nm], vnm = s * u[(1 + (f >> 1)) * Np + nm];
+        const TC pp = ss * (TC)gp[r];
+        const TC vnp = sv * s * (TC)gv[r];
+        sfl[t] = (zp[r] * (vnp - vnm) + (pm - pp)) / (zm[r] + zp[r]);
+      }
     }
-  }
-  __syncthreads();
-  TC *sfl = sq; /* [EPB][4][Nfp] */
-#pragma unroll
-  for (int r = 0; r < TPT; ++r)
-  {
-    const int t = tid + r * BS;
-    if (tid < BS && t < NT && t / (4 * Nfp) < tk.ne)
-      sfl[t] = fl[r];
-  }
-  __syncthreads();
+    __syncthreads();
 
-  if (act)
-  {
-    gptr<const TC> G = geo_tab<TC>(sd) + (size_t)e * GEO_STRIDE;
-    const TC *F = sfl + le * 4 * Nfp;
+    if (act)
+    {
+      const TC *F = sfl + le * 4 * Nfp;
 #define BFAMX_ALIFT(face, cond, fn_)                                           \
   if (cond)                                                                    \
   {                                                                            \
-    const TC lift = G[GEO_LX + ((face) >> 1)];                                 \
+    const TC lift = (face) < 2 ? lx : ly;                                      \
     const TC dvn = F[(face)*Nfp + (fn_)];                                      \
     const TC sg = ((face)&1) ? TC(1) : TC(-1);                                 \
     rate[1 + ((face) >> 1)] += lift * Zm * dvn * sg * rhoi;                    \
     rate[0] -= lift * bulk * dvn;                                              \
   }
-    BFAMX_ALIFT(0, i == 0, j)
-    BFAMX_ALIFT(1, i == N, j)
-    BFAMX_ALIFT(2, j == 0, i)
-    BFAMX_ALIFT(3, j == N, i)
+      BFAMX_ALIFT(0, i == 0, j)
+      BFAMX_ALIFT(1, i == N, j)
+      BFAMX_ALIFT(2, j == 0, i)
+      BFAMX_ALIFT(3, j == N, i)
 #undef BFAMX_ALIFT
-  }
-
+    }
   }
   if (!act)
     return;
@@ -180,36 +230,22 @@ __device__ __forceinline__ void acoustic_task(const SD &sd, const Task &tk,
       rate[f] += w * (TC)sd.src_amp[f] * g;
   }
 
-  if (la.mode == MODE_RHS || PART != PART_FUSED)
+  if (!upd)
   {
 #pragma unroll
     for (int f = 0; f < NF; ++f)
       glob(sd.rhs)[qidx(e, f, n, NF, Np)] = (double)rate[f];
     return;
   }
-  gptr<TS> qout = glob(static_cast<TS *>(sd.q[cx.parity ^ 1]));
-  gptr<TR> dqp = glob(static_cast<TR *>(sd.dq));
   const TR ca = (TR)cx.a, cdt = (TR)cx.dt;
   const TS cb = (TS)cx.b;
-  /* A = 0 (first stage of a step): no dq read.  FP32, FP64: the old dq is
-   * rebuilt from the previous state, B_{s-1} dq_{s-1} = q_s - q_{s-1},
-   * read from the other ping-pong buffer before this thread overwrites the
-   * node (a holds A_s / B_{s-1}) */
-  const bool rd_dq = cx.a != 0.0;
-  constexpr bool REC = sizeof(TS) == sizeof(TR);
-  const bool rec = REC && cx.rec;
 #pragma unroll
   for (int f = 0; f < NF; ++f)
   {
     const size_t id = qidx(e, f, n, NF, Np);
     TR dqo = 0;
     if (rd_dq)
-    {
-      if constexpr (REC)
-        dqo = rec ? (TR)(qs[f] - qout[id]) : dqp[id];
-      else
-        dqo = dqp[id];
-    }
+      dqo = rec ? (TR)qs[f] - old[f] : old[f];
     const TR d = ca * dqo + cdt * (TR)rate[f];
     if (!cx.dq_dead && !rec)
       dqp[id] = d;
@@ -225,12 +261,35 @@ acoustic_stage_kernel(LaunchArgs a)
   const TaskWalk w = task_walk(a, a.ntasks);
   for (int v = w.first; v < w.end; v += w.stride)
   {
-    const Task tk = load_task(a.tasks, task_at(a, a.ntasks, v));
+    const Task tk = launch_task<EPB, true>(a, task_at(a, a.ntasks, v));
     const auto &sd = *(cglob(a.subs) + tk.sub);
-    const StageCtx cx = stage_ctx(sd, a);
+    const StageCtx cx = stage_ctx<true>(sd, a);
     acoustic_task<N, EPB, P>(sd, tk, cx, a, smem);
     __syncthreads();
   }
+}
+
+/* Blocks of up to 256 threads; of one wavefront for one subdomain (its tasks
+ * are then computed) of at most SMALL_TASKS such tasks, which spreads it over
+ * more CUs and leaves its barriers nothing to wait for.  us per stage, FP64,
+ * 256 / 64 threads: N = 4 XXX */
+constexpr int SMALL_TASKS = 128;
+
+template <int N, class P>
+static hipError_t launch_ae(const LaunchArgs &a, int grid, hipStream_t s)
+{
+  constexpr int Np = (N + 1) * (N + 1), E = 256 / Np, S = 64 / Np < 1 ? 1 : 64 / Np;
+  if (a.one && a.ntasks <= SMALL_TASKS)
+  {
+    LaunchArgs b = a;
+    b.ntasks = (a.one_K + S - 1) / S;
+    const int nx = a.xcd_remap == 1 && a.nxcd > 1 ? a.nxcd : 1;
+    hipLaunchKernelGGL((acoustic_stage_kernel<N, S, P>), dim3(nx * ((b.ntasks + nx - 1) / nx)),
+                       dim3(S * Np), 0, s, b);
+  }
+  else
+    hipLaunchKernelGGL((acoustic_stage_kernel<N, E, P>), dim3(grid), dim3(E * Np), 0, s, a);
+  return hipGetLastError();
 }
 
 template <class P>
@@ -239,13 +298,7 @@ static hipError_t launch_an(int N, const LaunchArgs &a, int grid, hipStream_t s)
   switch (N)
   {
 #define BFAMX_CASE(NN)                                                         \
-  case NN:                                                                     \
-  {                                                                            \
-    constexpr int E = 256 / ((NN + 1) * (NN + 1));                             \
-    hipLaunchKernelGGL((acoustic_stage_kernel<NN, E, P>), dim3(grid),          \
-                       dim3(E * (NN + 1) * (NN + 1)), 0, s, a);                \
-    break;                                                                     \
-  }
+  case NN: return launch_ae<NN, P>(a, grid, s);
     BFAMX_CASE(1)
     BFAMX_CASE(2)
     BFAMX_CASE(3)
