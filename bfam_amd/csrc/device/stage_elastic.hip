@@ -34,7 +34,6 @@
  * The task, descriptor, clock and, for one-element blocks, the element
  * tables are read through the constant address space (scalar loads).
  */
-#include <climits>
 #include <type_traits>
 
 #include "elastic_axis.hpp"
@@ -74,12 +73,15 @@ template <int N> struct NodeFaceLift
  * N = 6 FP32 rates 420 / 391 (28^3), 96 / 91 (17^3); N = 5 (36 of 64 lanes,
  * six units on four wavefronts, one block per element) FP64 340 / 306 (32^3),
  * 67.3 / 60.6 (18^3), FP32 297 / 292 (38^3), 54.8 / 53.9 (21^3), but FP32 rates
- * 59.7 / 63.2 (18^3). */
+ * 59.7 / 63.2 (18^3); N = 4 (25 of 64 lanes, six units on two wavefronts; as tasks
+ * 25 of its 150 face nodes run a second round, and registers spill) FP32 78.2 /
+ * 66.6 (27^3), 394 / 321 (46^3), FP64 59.7 / 52.2 (20^3), but FP32 rates 55.1 / 63.1
+ * (20^3). */
 template <int N, int EPB, class P> struct NodeUnits
 {
   static constexpr bool rates32 = __is_same(P, P32R);
   static constexpr bool value =
-      EPB == 1 && !P::MF && (N == 7 || (N == 6 && rates32) || (N == 5 && !rates32));
+      EPB == 1 && !P::MF && (N == 7 || (N == 6 && rates32) || ((N == 4 || N == 5) && !rates32));
 };
 
 /* threads of a block: its volume nodes, and for face units whole wavefronts */
@@ -878,14 +880,12 @@ template <int N, class P> struct NodeEpbAlt
  * 0.523-0.530.  us per stage, whole tasks / split: N = 5 FP32 316 / 297 (38^3),
  * 58.9 / 54.8 (21^3), 12.4 / 10.2 (10^3), 10.4 / 7.3 (6^3), FP32 rates 260 / 257
  * (30^3), 64.2 / 59.6 (18^3), 12.8 / 8.7 (8^3), FP64 364 / 340 (32^3), 69.6 / 67.3
- * (18^3), 12.9 / 9.3 (8^3); FP64 N = 4 (12 bytes of spill per lane) 23.3 /
- * 7.7 (4^3), 61.6 / 59.8 (20^3), 164 / 156 (28^3), but 290 / 304 (34^3): whole
- * tasks from max_tasks on. */
+ * (18^3), 12.9 / 9.3 (8^3); FP64 N = 4 23.3 / 7.6 (4^3), with face units 257 /
+ * 230 (34^3). */
 template <int N, int EPB, class P> struct NodeSplit
 {
   static constexpr int TE = 512 / ((N + 1) * (N + 1) * (N + 1)) < 1 ? 1 : 512 / ((N + 1) * (N + 1) * (N + 1));
   static constexpr int value = !P::MF && EPB == NodeEpb<N, P>::value ? TE / EPB : 1;
-  static constexpr int max_tasks = N == 4 && __is_same(P, P64) ? 7168 : INT_MAX;
 };
 
 /* blocks per XCD and cube in the block order of the fused kernel (mode 2 of
@@ -981,17 +981,22 @@ static hipError_t launch_ne(const LaunchArgs &a, int grid, hipStream_t s, unsign
 {
   constexpr int NS = NodeSplit<N, EPB, P>::value;
   /* EPB elements per block, or, on a resident grid (fewer blocks than
-   * tasks), per turn of a block */
+   * tasks), per turn of a block.  A split order's turns are short and its
+   * resident grid is eight times the blocks that fit, so that a CU's next
+   * blocks start while others still run their turn (us per stage, FP32 N = 4
+   * with one time, two, four, eight, and a block per element: 71.2, 69.7,
+   * 67.2, 66.6, 66.6 (27^3); 348, 346, 337, 328, 321 (46^3)) */
   if constexpr (NS > 1)
-    if (a.ntasks < NodeSplit<N, EPB, P>::max_tasks)
-    {
-      const int vt = a.ntasks * NS;
-      if (grid >= a.ntasks)
-        grid = a.xcd_remap == 1 && a.nxcd > 1 ? a.nxcd * ((vt + a.nxcd - 1) / a.nxcd) : vt;
-      hipLaunchKernelGGL((elastic_stage_kernel<N, EPB, P, true>), dim3(grid),
-                         dim3(NodeBlock<N, EPB, P>::value), dyn, s, a);
-      return hipGetLastError();
-    }
+  {
+    const int vt = a.ntasks * NS;
+    if (grid >= a.ntasks)
+      grid = a.xcd_remap == 1 && a.nxcd > 1 ? a.nxcd * ((vt + a.nxcd - 1) / a.nxcd) : vt;
+    else
+      grid = grid < vt / 8 ? 8 * grid : vt;
+    hipLaunchKernelGGL((elastic_stage_kernel<N, EPB, P, true>), dim3(grid),
+                       dim3(NodeBlock<N, EPB, P>::value), dyn, s, a);
+    return hipGetLastError();
+  }
   hipLaunchKernelGGL((elastic_stage_kernel<N, EPB, P>), dim3(grid),
                      dim3(NodeBlock<N, EPB, P>::value), dyn, s, a);
   return hipGetLastError();

@@ -1,7 +1,7 @@
 """The node-parallel stage at the edges of its launch forms: block orders
 (device tuning 0, 1, 2), one block per element, per task and resident grids
-give the same bits, at element counts around a task, a cube of 64 tasks, a
-group of 512 and, FP64 N = 4, where blocks take whole tasks."""
+give the same bits, at element counts around a task, a cube of 64 tasks
+and a group of 512."""
 import numpy as np
 import pytest
 
@@ -39,19 +39,3 @@ def test_launch_forms_agree(n, N, prec):
     assert np.isfinite(ref).all() and np.abs(ref - q0).max() > 0
     for kind, remap in ((1, 1), (1, 2), (2, 0), (2, 1), (2, 2)):
         np.testing.assert_array_equal(_final(cfg, q0, prec, N, kind, remap), ref)
-
-
-@pytest.mark.parametrize("nx", [28, 27])
-def test_fp64_n4_whole_and_split_tasks(nx):
-    """7168 tasks of four elements take whole tasks, 6912 one block per
-    element; the two forms compute an element alike up to the rounding of a
-    differently contracted sum (states of order 1, ten stages: 1e-13)."""
-    N = 4
-    mesh = W.Mesh(3, [nx, 32, 32], N, L=[1.0, 1.0, 1.0])
-    assert (mesh.K >= 4 * 7168) == (nx == 28)
-    cfg, q0 = random_elastic((nx, 32, 32), N, seed=nx)
-    a = _final(cfg, q0, bx.FP64, N, 1, 2)
-    b = _final(cfg, q0, bx.FP64, N, 3, 2)
-    scale = np.abs(a).max()
-    assert np.isfinite(a).all()
-    assert np.abs(a - b).max() <= 1e-13 * scale
