@@ -106,7 +106,8 @@ struct bfamx_device
    * bfamx_batch_autotune: -1 unknown (the default of the per-order
    * measurements), 0 line (one wavefront per element, lanes own lines), 1
    * node-parallel (threads own nodes), 2 node-parallel on a resident grid
-   * (as many blocks as fit the CUs at once, each looping over tasks), 3 and
+   * (as many blocks as fit the CUs at once, or eight times that at the orders
+   * that split their tasks, each looping over tasks), 3 and
    * 4 as 1 and 2 with the kernel's other block size (N = 3..5) */
   signed char kchoice[NPREC][9];
   /* resident-block cap per precision, order and kernel slot (0 line, 1
@@ -1185,11 +1186,10 @@ static int grid_for(const bfamx_device_t *d, int ntasks)
 
 /* the stage kernel of an order not (yet) autotuned (0 line, 1
  * node-parallel, 2 node-parallel on a resident grid): the one measured
- * fastest, us per stage with one block per task / on the resident grid:
- * FP32 N=4 78.5 / 95.0 (27^3) and 394 / 437 (46^3), N=5 316 / 333 (38^3),
- * N=6 64.0 / 63.2 (18^3) and 346 / 325 (32^3), N=7 374 / 410 (32^3); FP64
- * N=5 351 / 366 (32^3), N=6 91 / 82 (16^3) and 380 / 336 (26^3), N=7 90 / 101
- * (16^3) and 374 / 420 (26^3); FP32 rates N=6 420 / 562 (28^3) */
+ * fastest, us per stage with one block per task (or element) / on the
+ * resident grid: FP32 N=4 66.6 / 66.6 (27^3) and 321 / 328 (46^3), N=6 63.5 /
+ * 57.9 (18^3) and 341 / 316 (32^3); FP64 N=4 52.2 / 52.2 (20^3), N=6 89.4 / 75.8
+ * (16^3), N=7 420 / 391 (26^3) */
 static int default_kind(int prec, int N)
 {
   switch (prec)

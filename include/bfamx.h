@@ -361,7 +361,8 @@ int bfamx_timer_stop(bfamx_device_t *dev, float *ms);
 /* launch tuning, the order in which blocks take elements: 0 hardware
  * round-robin over the XCDs, 1 a contiguous element range per XCD, 2 (the
  * default, measured fastest) one round-robin front with each XCD taking
- * whole 2x2x2 Morton cubes, so that their inner faces share an L2 */
+ * whole Morton cubes (4x4x4 tasks of the node-parallel stage, 2x2x2 of the
+ * others), so that their inner faces share an L2 */
 int bfamx_set_tuning(bfamx_device_t *dev, int xcd_remap);
 /* elastic stage launches: 1 at most the resident wavefronts, each looping
  * over tasks and streaming the next task's state into LDS while it writes
