@@ -870,8 +870,9 @@ template <int N, class P> struct NodeEpbAlt
 };
 
 /* blocks per node task on a one-block-per-task grid: the task's elements
- * over EPB (each block taking EPB of them) where that measured faster than
- * one block taking the whole task in passes, 1 elsewhere.  FP64 at N = 3
+ * over EPB (each block taking EPB of them) at the block size of NodeEpb, where
+ * it measured faster than one block taking the whole task in passes; 1 at
+ * the other block size and for the matrix-core derivatives.  FP64 at N = 3
  * (two-element blocks): 0.805 -> 0.789 ms per stage.  Each XCD's
  * blocks then cover 2x2x2 elements of a Morton group instead of 4x4x4
  * (N = 3), and fewer elements are in flight per XCD, and a small subdomain
