@@ -890,7 +890,7 @@ template <int N, int EPB, class P> struct NodeSplit
 };
 
 /* blocks per XCD and cube in the block order of the fused kernel (mode 2 of
- * first_task): 4 x 4 x 4 tasks.  A cube's inner faces are gathered from the
+ * task_at): 4 x 4 x 4 tasks.  A cube's inner faces are gathered from the
  * XCD's L2, its outer ones miss it by whole lines (an x face of N = 3 or 7
  * touches every line of its rows), and a quarter of the faces of a 4 x 4 x 4
  * cube are outer ones, against half with 2 x 2 x 2.  Read misses per stage,
