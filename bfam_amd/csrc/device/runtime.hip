@@ -1125,10 +1125,15 @@ extern "C" int bfamx_set_fields(bfamx_subdomain_t *s,
   return BFAMX_OK;
 }
 
-/* which buffer holds the state after the stages launched so far */
-static int current_parity(const bfamx_subdomain_t *s)
+/* which buffer holds the state, by the device's count of stages: a caller may
+ * capture stages on the device's stream, which runs none, and replay them,
+ * which the host does not see */
+static int current_parity(bfamx_subdomain_t *s, int *parity)
 {
-  return s->prec == BFAMX_FP64_PLAIN ? 0 : (int)(s->stages_run & 1);
+  ClockHead c;
+  int rc = read_clock(s, &c);
+  *parity = s->prec == BFAMX_FP64_PLAIN ? 0 : (int)(c.stage & 1);
+  return rc;
 }
 
 extern "C" int bfamx_get_time(bfamx_subdomain_t *s, double *t, int64_t *stages)
@@ -1153,7 +1158,9 @@ extern "C" int bfamx_download_fields(bfamx_subdomain_t *s,
     return bfamx_fail(BFAMX_EINVAL, "bfamx_download_fields: NULL argument");
   if (!s->fields_set)
     return bfamx_fail(BFAMX_ESTATE, "bfamx_download_fields: no state set");
-  const int parity = current_parity(s);
+  int parity, rc = current_parity(s, &parity);
+  if (rc)
+    return rc;
   return s->state_fp32 ? copy_fields<float, true>(s, s->h.q[parity], fields)
                        : copy_fields<double, true>(s, s->h.q[parity], fields);
 }
@@ -1512,7 +1519,10 @@ extern "C" int bfamx_reduce_energy(bfamx_subdomain_t *s, double *energy)
 {
   if (!s || !energy)
     return bfamx_fail(BFAMX_EINVAL, "bfamx_reduce_energy: NULL argument");
-  hipError_t e = launch_energy(s->h, s->state_fp32, current_parity(s), s->d_partial,
+  int parity, rc = current_parity(s, &parity);
+  if (rc)
+    return rc;
+  hipError_t e = launch_energy(s->h, s->state_fp32, parity, s->d_partial,
                                s->dev->stream);
   if (e != hipSuccess)
     return bfamx_fail(BFAMX_EHIP, "energy launch: %s", hipGetErrorString(e));
@@ -1548,8 +1558,10 @@ extern "C" int bfamx_reduce_l2_diff(bfamx_subdomain_t *a, bfamx_subdomain_t *b,
     return bfamx_fail(BFAMX_EINVAL, "bfamx_reduce_l2_diff: NULL argument");
   if (a->K != b->K || a->N != b->N || a->physics != b->physics || a->dev != b->dev)
     return bfamx_fail(BFAMX_EINVAL, "bfamx_reduce_l2_diff: different shapes");
-  hipError_t e = launch_l2diff(a->h, a->state_fp32, current_parity(a), b->h, b->state_fp32,
-                               current_parity(b),
+  int pa, pb, rc = current_parity(a, &pa);
+  if (rc || (rc = current_parity(b, &pb)))
+    return rc;
+  hipError_t e = launch_l2diff(a->h, a->state_fp32, pa, b->h, b->state_fp32, pb,
                                a->d_partial, a->dev->stream);
   if (e != hipSuccess)
     return bfamx_fail(BFAMX_EHIP, "l2diff launch: %s", hipGetErrorString(e));
@@ -2501,9 +2513,12 @@ extern "C" int bfamx_batch_autotune(bfamx_batch_t *b, int trials, int force,
     reg[i] = s->h.dq;
     if (s->h.dq_rec)
     {
-      reg[i] = s->h.q[current_parity(s) ^ 1];
+      int parity = 0;
+      rc = current_parity(s, &parity);
+      reg[i] = s->h.q[parity ^ 1];
     }
-    rc = dev_alloc(d, allocs, &bytes, nb, &saved[i]);
+    if (!rc)
+      rc = dev_alloc(d, allocs, &bytes, nb, &saved[i]);
     if (!rc && hipMemcpyAsync(saved[i], reg[i], nb, hipMemcpyDeviceToDevice, d->stream) !=
                    hipSuccess)
       rc = bfamx_fail(BFAMX_EHIP, "autotune: dq save failed");
@@ -2856,7 +2871,10 @@ extern "C" int bfamx_transfer_fields(const bfamx_transfer_maps_t *m,
   std::vector<XferSide> hs(nsrc), hd(ndst);
   for (int i = 0; i < nsrc; ++i)
   {
-    hs[i].q = src[i]->h.q[current_parity(src[i])];
+    int parity = 0, rc = current_parity(src[i], &parity);
+    if (rc)
+      return rc;
+    hs[i].q = src[i]->h.q[parity];
     hs[i].N = src[i]->N;
     hs[i].K = src[i]->K;
   }
