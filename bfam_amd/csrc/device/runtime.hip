@@ -160,6 +160,9 @@ struct bfamx_subdomain
   /* whose descriptor's source and forcing the clock's slots were computed
    * with: the subdomain's own (0), or the copy of the batch of that id */
   unsigned long long clock_by;
+  /* stages were captured by the caller: replays, which the host does not
+   * see, may have computed the slots with other descriptors */
+  bool clock_replayed;
   bfamx_lsrk_t lsrk;
   bfamx_glue_t *glue; /* set while faces of this subdomain are glued */
 };
@@ -555,18 +558,24 @@ static int set_clock(bfamx_subdomain_t *s, double t0, double dt)
 /* before a run of stages from the n descriptors d_subs of the members (`by`:
  * as clock_by): slots that another descriptor computed are recomputed with
  * these, except the stage about to run, whose parameters the clock's last
- * advance fixed */
+ * advance fixed.  In a caller's capture, whose replays may follow any other
+ * run, always */
 static int own_clocks(bfamx_device_t *d, bfamx_subdomain_t *const *subs, int n,
                       const SubDev *d_subs, unsigned long long by)
 {
+  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+  HIPCHK(hipStreamIsCapturing(d->stream, &capture));
   bool all = true;
   for (int i = 0; i < n; ++i)
   {
-    all = all && subs[i]->clock_by == by;
-    subs[i]->clock_by = by;
+    subs[i]->clock_replayed |= capture != hipStreamCaptureStatusNone;
+    all = all && subs[i]->clock_by == by && !subs[i]->clock_replayed;
   }
-  if (!all)
-    HIPCHK(launch_clock_advance(d_subs, n, 0, 1, d->stream));
+  if (all)
+    return BFAMX_OK;
+  HIPCHK(launch_clock_advance(d_subs, n, 0, 1, d->stream));
+  for (int i = 0; i < n; ++i)
+    subs[i]->clock_by = by;
   return BFAMX_OK;
 }
 

@@ -1,6 +1,8 @@
 """Stages captured by the caller on the device's stream (bfamx_device_stream)
 and replayed there: the capture itself runs none, and every query afterwards
-sees the stages replayed, an odd number of them included."""
+sees the stages replayed, an odd number of them included.  Replays mix with
+eager runs of the same subdomain through other descriptors: a batch keeps
+those of its creation, and a later source is the subdomain's own."""
 import ctypes as C
 
 import numpy as np
@@ -95,5 +97,41 @@ def test_batch_captured_by_the_caller(prec):
             r.step(2)
     g.close()
     for x in (b, r, *subs, *refs):
+        x.close()
+    dev.close()
+
+
+@pytest.mark.parametrize("replayed", ["subdomain", "batch"])
+@pytest.mark.parametrize("acoustic", [False, True], ids=["elastic", "acoustic"])
+def test_replays_mix_with_runs_of_other_descriptors(acoustic, replayed):
+    print(f"mixed descriptors acoustic={acoustic} replayed={replayed}", flush=True)
+    dev = bx.Device(0)
+
+    def state():
+        cfg, q0 = random_acoustic((3, 2), 4, 3) if acoustic else random_elastic((2, 1, 2), 4, 3)
+        src = dict(cfg["src"], t0=6 * cfg["dt"], f0=0.02 / cfg["dt"])
+        cfg["src"] = src
+        s = W.upload(dev, cfg, bx.FP64)
+        b = bx.Batch(dev, [s])
+        # the subdomain's own source from here on
+        s.set_source(src["elem"], src["weights"], [3.0 * a for a in src["amp"]],
+                     2.3 * src["f0"], src["t0"])
+        s.set_fields(q0, 0.0, cfg["dt"])
+        return s, b
+
+    sub, batch = state()
+    ref, rbatch = state()
+    own, other = (sub.step, batch.step) if replayed == "subdomain" else (batch.step, sub.step)
+    rown, rother = (ref.step, rbatch.step) if replayed == "subdomain" else (rbatch.step, ref.step)
+    g = Capture(dev, own)
+    for turn in range(6):
+        g.launch()
+        rown()
+        if turn % 3 != 1:
+            other(1 + turn % 2)
+            rother(1 + turn % 2)
+        np.testing.assert_array_equal(sub.download(), ref.download())
+    g.close()
+    for x in (batch, rbatch, sub, ref):
         x.close()
     dev.close()
