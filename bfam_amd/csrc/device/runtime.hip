@@ -987,13 +987,16 @@ extern "C" int bfamx_set_forcing_mms(bfamx_subdomain_t *s, double k,
   return refresh_clock(s);
 }
 
-/* elements [e0, e1) of a [K][nf][Np] array of T (buf: from e0 on) to or from
- * bfam's per-field host arrays */
+/* Elements [e0, e1) of a [K][nf][Np] array of T (buf: from e0 on) to or from
+ * bfam's per-field host arrays, in buf's order: a piece that the device has
+ * just written is not in the host's caches, and read in strides it waits for
+ * each (right-hand sides out, us: 0.56 MB 82 field by field, 61 in order;
+ * 0.84 MB 111, 72; 1.97 MB 202, 124) */
 template <class T, bool OUT, class F>
 static void host_rows(T *buf, F *const *fields, size_t e0, size_t e1, size_t nf, size_t Np)
 {
-  for (size_t f = 0; f < nf; ++f)
-    for (size_t e = e0; e < e1; ++e)
+  for (size_t e = e0; e < e1; ++e)
+    for (size_t f = 0; f < nf; ++f)
     {
       T *b = buf + ((e - e0) * nf + f) * Np;
       F *h = fields[f] + e * Np;
