@@ -1027,11 +1027,12 @@ static int copy_fields(bfamx_subdomain_t *s, void *dev_array, F *const *fields)
   const size_t Np = s->Np, nf = s->nf, K = s->K;
   const size_t per = nf * Np * sizeof(T), total = K * per;
   std::lock_guard<std::mutex> lock(d->fc.mu);
-  /* one thread below 2 MB out and 4 MB in (in / out by one and by four
-   * threads: 1.2 MB 70 / 171 and 107 / 125 us, 2.3 MB 128 / 261 and 146 / 162,
-   * 7.8 MB 641 / 1082 and 313 / 393), and the first copy on another stream
-   * after an allocation waits 0.8 ms for it; then one per MiB, with pieces of
-   * at least 256 KiB (at most a buffer) so that each worker has two or more */
+  /* one thread below 2 MB out and 4 MB in (us by one / four threads, in: 1.1 MB
+   * 70 / 80, 2.2 MB 118 / 113, 4.4 MB 205 / 148; right-hand sides out: 1.1 MB
+   * 88 / 84, 2.2 MB 152 / 124, 7.7 MB 413 / 254), and the first copy on another
+   * stream after an allocation waits 0.8 ms for it; then one per MiB, with
+   * pieces of at least 256 KiB (at most a buffer) so that each worker has two
+   * or more */
   const size_t mib = total >> 20;
   const int nw = mib < (OUT ? 2 : 4) ? 1 : mib < FC_WORKERS ? (int)mib : FC_WORKERS;
   size_t bytes = total / (2 * nw);
