@@ -20,7 +20,6 @@
 #include <algorithm>
 #include <atomic>
 #include <mutex>
-#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -1076,13 +1075,12 @@ static int copy_fields(bfamx_subdomain_t *s, void *dev_array, F *const *fields)
   else
   {
     HIPCHK(hipStreamSynchronize(d->stream));
-    std::vector<std::thread> th;
-    th.reserve(nw);
+    std::thread th[FC_WORKERS];
     for (int i = 1; i < nw; ++i)
     {
       try
       {
-        th.emplace_back([&, i] {
+        th[i] = std::thread([&, i] {
           const hipError_t e = hipSetDevice(d->hip_dev);
           if (e != hipSuccess)
             err = e;
@@ -1090,14 +1088,15 @@ static int copy_fields(bfamx_subdomain_t *s, void *dev_array, F *const *fields)
             work(i, d->fc.st[i]);
         });
       }
-      catch (const std::system_error &)
+      catch (...)
       {
-        break; /* no more threads: those that run take the pieces */
+        break; /* no more threads or memory: those that run take the pieces */
       }
     }
     work(0, d->fc.st[0]);
     for (std::thread &t : th)
-      t.join();
+      if (t.joinable())
+        t.join();
   }
   if (err != hipSuccess)
     return bfamx_fail(BFAMX_EHIP, "field copy failed: %s",
