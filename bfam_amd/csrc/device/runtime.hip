@@ -40,8 +40,8 @@ struct FieldCopy
   char *buf[FC_WORKERS] = {};
   bool pinned[FC_WORKERS] = {};
   hipStream_t st[FC_WORKERS] = {};
-  /* the buffer and stream of worker i */
-  hipError_t get(int i)
+  /* the buffer and, if `own`, the stream of worker i */
+  hipError_t get(int i, bool own)
   {
     if (!buf[i])
     {
@@ -56,7 +56,7 @@ struct FieldCopy
         return hipErrorOutOfMemory;
       buf[i] = (char *)p;
     }
-    return st[i] ? hipSuccess : hipStreamCreateWithFlags(&st[i], hipStreamNonBlocking);
+    return st[i] || !own ? hipSuccess : hipStreamCreateWithFlags(&st[i], hipStreamNonBlocking);
   }
   ~FieldCopy()
   {
@@ -1033,7 +1033,7 @@ static int copy_fields(bfamx_subdomain_t *s, void *dev_array, F *const *fields)
    * pieces of at least 256 KiB (at most a buffer) so that each worker has two
    * or more */
   const size_t mib = total >> 20;
-  const int nw = mib < (OUT ? 2 : 4) ? 1 : mib < FC_WORKERS ? (int)mib : FC_WORKERS;
+  int nw = mib < (OUT ? 2 : 4) ? 1 : mib < FC_WORKERS ? (int)mib : FC_WORKERS;
   size_t bytes = total / (2 * nw);
   bytes = bytes < ((size_t)256 << 10) ? (size_t)256 << 10 : bytes > FC_BYTES ? FC_BYTES : bytes;
   if (nw == 1)
@@ -1043,7 +1043,17 @@ static int copy_fields(bfamx_subdomain_t *s, void *dev_array, F *const *fields)
   HIPCHK(hipGetDevice(&dev0));
   hipError_t ge = hipSetDevice(d->hip_dev);
   for (int i = 0; i < nw && ge == hipSuccess; ++i)
-    ge = d->fc.get(i);
+  {
+    ge = d->fc.get(i, nw > 1);
+    if (ge != hipSuccess && nw > 1)
+    {
+      /* no more buffers or streams: the workers that have theirs copy, one
+       * alone on the device's stream */
+      (void)hipGetLastError();
+      nw = i > 1 ? i : 1;
+      ge = d->fc.get(0, false);
+    }
+  }
   (void)hipSetDevice(dev0);
   HIPCHK(ge);
   std::atomic<size_t> next{0};
