@@ -537,10 +537,12 @@ static int read_clock(bfamx_subdomain_t *s, ClockHead *c)
   return BFAMX_OK;
 }
 
-/* recompute the parameters of the stages about to run, after the clock or
- * the subdomain's descriptor changed */
+/* recompute the parameters of the stages about to run, after the subdomain's
+ * descriptor changed; before there is a state, set_clock will fill them */
 static int refresh_clock(bfamx_subdomain_t *s)
 {
+  if (!s->fields_set)
+    return BFAMX_OK;
   s->clock_by = 0;
   HIPCHK(launch_clock_advance(s->d_sub, 1, 0, 0, s->dev->stream));
   return BFAMX_OK;
@@ -859,9 +861,7 @@ extern "C" int bfamx_subdomain_upload(bfamx_device_t *dev,
       goto fail;
     }
   }
-  rc = push_sub(s);
-  if (!rc)
-    rc = refresh_clock(s);
+  rc = push_sub(s); /* the clock's slots are filled by set_clock */
   if (rc)
     goto fail;
   *out = s;
