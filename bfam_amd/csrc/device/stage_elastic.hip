@@ -722,10 +722,22 @@ __device__ __forceinline__ void elastic_task(const SD &sd, const Task &tk,
     /* one wavefront meets all six faces: one branch per axis, for the face
      * of the axis the node lies on, runs three lifts instead of six.  us per
      * stage, six branches / three: 50.2 / 49.2 (30^3), 289 / 284 (56^3), 6.17 /
-     * 6.05 (8^3); FP32 N = 6 then takes over 96 scalar registers (NodeWaves) */
+     * 6.05 (8^3); FP32 N = 6 then takes over 96 scalar registers (NodeWaves).
+     * The sign is a run-time value here, and on face 0 the other product of
+     * lambda dvn + 2 mu dvn is rounded by itself: the results move by some
+     * 1e-7, their distance from FP64 does not (L2 after ten steps, six / three:
+     * 1.251e-7 / 1.253e-7 (6^3), 1.230e-7 / 1.230e-7 (13^3)).  With the products
+     * rounded as in six branches, three take 50.7 (30^3) and 293 (56^3) */
     const TC *F = sfl + le * 6 * FC * Nfp;
     TC flv[6];
-#define BFAMX_LIFT(A, c_, fn_)                                                   if ((c_) == 0 || (c_) == N)                                                    {                                                                                const TC *Ff = F + (2 * (A) + ((c_) == N)) * FC * Nfp + (fn_);                 _Pragma("unroll") for (int c = 0; c < 6; ++c) flv[c] = Ff[c * Nfp];            elastic_lift<TC>(A, (c_) == N ? TC(1) : TC(-1), G[GEO_LX + (A)], rhoi,                          lam, mu, flv, rate);                                        }
+#define BFAMX_LIFT(A, c_, fn_)                                                 \
+  if ((c_) == 0 || (c_) == N)                                                  \
+  {                                                                            \
+    const TC *Ff = F + (2 * (A) + ((c_) == N)) * FC * Nfp + (fn_);             \
+    _Pragma("unroll") for (int c = 0; c < 6; ++c) flv[c] = Ff[c * Nfp];        \
+    elastic_lift<TC>(A, (c_) == N ? TC(1) : TC(-1), G[GEO_LX + (A)], rhoi,     \
+                     lam, mu, flv, rate);                                      \
+  }
     BFAMX_LIFT(0, i, j + n1 * k)
     BFAMX_LIFT(1, j, i + n1 * k)
     BFAMX_LIFT(2, k, i + n1 * j)
@@ -1100,7 +1112,7 @@ hipError_t launch_elastic_plain(int N, const LaunchArgs &a, int grid,
     hipLaunchKernelGGL((elastic_part_kernel<NN, EE, PART_VOLUME>), dim3(grid), \
                        dim3(NodeBlock<NN, EE, P64>::value), 0, s, a);          \
     hipLaunchKernelGGL((elastic_part_kernel<NN, EE, PART_SURFACE>),            \
-                       dim3(grid), dim3(NodeBlock<NN, EE, P64>::value), 0, s, a);                                               \
+                       dim3(grid), dim3(NodeBlock<NN, EE, P64>::value), 0, s, a); \
     break;
     BFAMX_CASE(3, 8)
     BFAMX_CASE(4, 4)
