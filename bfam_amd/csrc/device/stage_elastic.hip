@@ -987,8 +987,7 @@ elastic_stage_kernel(LaunchArgs a)
 }
 
 /* the launch of order N with EPB elements per block, or the occupancy
- * calculator's resident blocks per CU for it (of the whole-task form: a split
- * order's has its registers or fewer) */
+ * calculator's resident blocks per CU for the kernel that it launches */
 template <int N, int EPB, class P>
 static hipError_t launch_ne(const LaunchArgs &a, int grid, hipStream_t s, unsigned dyn)
 {
@@ -1018,7 +1017,8 @@ template <int N, int EPB, class P>
 static hipError_t occupancy_ne(int *blocks, unsigned dyn)
 {
   return hipOccupancyMaxActiveBlocksPerMultiprocessor(
-      blocks, elastic_stage_kernel<N, EPB, P>, NodeBlock<N, EPB, P>::value, dyn);
+      blocks, elastic_stage_kernel<N, EPB, P, (NodeSplit<N, EPB, P>::value > 1)>,
+      NodeBlock<N, EPB, P>::value, dyn);
 }
 
 /* alt: the block size of NodeEpbAlt instead of NodeEpb */
