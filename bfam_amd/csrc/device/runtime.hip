@@ -105,7 +105,7 @@ struct bfamx_device
    * bfamx_batch_autotune: -1 unknown (the default of the per-order
    * measurements), 0 line (one wavefront per element, lanes own lines), 1
    * node-parallel (threads own nodes), 2 node-parallel on a resident grid
-   * (as many blocks as fit the CUs at once, or eight times that at the orders
+   * (as many blocks as fit the CUs at once, or 16 times that at the orders
    * that split their tasks, each looping over tasks), 3 and
    * 4 as 1 and 2 with the kernel's other block size (N = 3..5) */
   signed char kchoice[NPREC][9];
@@ -1214,11 +1214,12 @@ static int grid_for(const bfamx_device_t *d, int ntasks)
 }
 
 /* the stage kernel of an order not (yet) autotuned (0 line, 1
- * node-parallel, 2 node-parallel on a resident grid): the one measured
- * fastest, us per stage with one block per task (or element) / on the
- * resident grid: FP32 N=4 66.6 / 66.6 (27^3) and 321 / 328 (46^3), N=6 63.5 /
- * 57.9 (18^3) and 341 / 316 (32^3); FP64 N=4 52.2 / 52.2 (20^3), N=6 89.4 / 75.8
- * (16^3), N=7 420 / 391 (26^3) */
+ * node-parallel, 2 node-parallel on a resident grid): us per stage with one
+ * block per task (or element) / on the resident grid: FP32 N=6 63.5 / 57.9
+ * (18^3) and 341 / 316 (32^3); FP64 N=4 52.2 / 52.2 (20^3), N=6 89.4 / 75.8
+ * (16^3), N=7 420 / 391 (26^3).  FP32 N=4 are one grid up to some 45,000
+ * elements and within 1 % beyond (322 / 322 at 46^3, 580 / 579 at 56^3, 941 /
+ * 948 at 66^3) */
 static int default_kind(int prec, int N)
 {
   switch (prec)

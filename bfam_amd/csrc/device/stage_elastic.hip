@@ -986,6 +986,8 @@ elastic_stage_kernel(LaunchArgs a)
   }
 }
 
+constexpr int SPLIT_TURNS = 16;
+
 /* the launch of order N with EPB elements per block, or the occupancy
  * calculator's resident blocks per CU for the kernel that it launches */
 template <int N, int EPB, class P>
@@ -994,17 +996,19 @@ static hipError_t launch_ne(const LaunchArgs &a, int grid, hipStream_t s, unsign
   constexpr int NS = NodeSplit<N, EPB, P>::value;
   /* EPB elements per block, or, on a resident grid (fewer blocks than
    * tasks), per turn of a block.  A split order's turns are short and its
-   * resident grid is eight times the blocks that fit, so that a CU's next
-   * blocks start while others still run their turn (us per stage, FP32 N = 4
-   * with one time, two, four, eight, and a block per element: 71.2, 69.7,
-   * 67.2, 66.6, 66.6 (27^3); 348, 346, 337, 328, 321 (46^3)) */
+   * resident grid is SPLIT_TURNS times the blocks that fit, so that a CU's
+   * next blocks start while others still run their turn (us per stage, FP32
+   * N = 4 with one time, two, four, eight, 16, 32, and a block per element:
+   * 348, 346, 337, 326, 322, 322, 322 (46^3); the last four at 66^3 970, 948, 948,
+   * 941, and at 30^3 with FP32 rates 174, 177, 177, 178; eight, 16, 32: FP32 N = 3
+   * 160, 152, 154 (46^3), FP64 N = 5 217, 211, 209 (28^3)) */
   if constexpr (NS > 1)
   {
     const int vt = a.ntasks * NS;
     if (grid >= a.ntasks)
       grid = a.xcd_remap == 1 && a.nxcd > 1 ? a.nxcd * ((vt + a.nxcd - 1) / a.nxcd) : vt;
     else
-      grid = grid < vt / 8 ? 8 * grid : vt;
+      grid = grid < vt / SPLIT_TURNS ? SPLIT_TURNS * grid : vt;
     hipLaunchKernelGGL((elastic_stage_kernel<N, EPB, P, true>), dim3(grid),
                        dim3(NodeBlock<N, EPB, P>::value), dyn, s, a);
     return hipGetLastError();
