@@ -272,10 +272,16 @@ acoustic_stage_kernel(LaunchArgs a)
   }
 }
 
-/* Blocks of up to 256 threads; of one wavefront for one subdomain (its tasks
- * are then computed) of at most SMALL_TASKS such tasks, which spreads it over
- * more CUs and leaves its barriers nothing to wait for.  us per stage, FP64,
- * 256 / 64 threads: N = 4 XXX */
+/* Blocks of up to 256 threads; for one subdomain (its tasks are then
+ * computed) of at most SMALL_TASKS such tasks, blocks of as many elements as
+ * one wavefront holds (N = 8: one element, 81 threads), which spreads it over
+ * more CUs: few wavefronts then meet at each barrier.  Past some 128 tasks
+ * the CUs are busy either way, and small blocks cost launches and repeated
+ * loads of D.  us per stage, large / small blocks at about 32, 126 and 256
+ * tasks: FP64 N = 2 4.92 / 4.55, 5.00 / 4.76, 5.09 / 5.26; N = 4 4.20 / 3.83,
+ * 4.31 / 4.14, 4.40 / 4.60; N = 7 3.85 / 3.68, 3.90 / 3.77, 3.99 / 4.15; N = 8
+ * 4.21 / 3.87, 4.29 / 4.23, 4.43 / 4.75; FP32 N = 4 4.16 / 3.76, 4.18 / 4.06,
+ * 4.26 / 4.26; N = 8 3.99 / 3.75, 4.03 / 3.96, 4.09 / 4.17 */
 constexpr int SMALL_TASKS = 128;
 
 template <int N, class P>
