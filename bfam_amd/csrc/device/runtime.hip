@@ -2554,10 +2554,10 @@ extern "C" int bfamx_batch_autotune(bfamx_batch_t *b, int trials, int force,
   a.mode = MODE_STAGE;
   a.xcd_remap = d->xcd_remap;
   a.nxcd = d->num_xcd;
-  /* each trial launch starts from the saved buffers: a launch rewrites
-   * what the next one would read (dq, or the previous state that the
-   * rebuilt dq comes from), and without the restore the timed data would
-   * grow by |A_s| (or |B_s A_s / B_{s-1}|) per launch */
+  /* each trial starts from the saved buffers: a launch rewrites what the
+   * next one would read (dq, or the previous state that the rebuilt dq comes
+   * from), and without the restore the timed data would grow by |A_s| (or
+   * |B_s A_s / B_{s-1}|) per launch */
   auto restore = [&]() -> hipError_t {
     for (size_t i = 0; i < b->subs.size(); ++i)
       if (saved[i])
@@ -2646,11 +2646,14 @@ extern "C" int bfamx_batch_autotune(bfamx_batch_t *b, int trials, int force,
     for (int mode = 0; mode < 2 && !rc; ++mode)
     {
       b->grouped = mode;
+      /* a step's stages between one fork and one join, as a run has them at
+       * the least: with a fork and a join around each stage the launches per
+       * order looked slower than they run (93 against 62 us, batch_chains) */
       rc = time_it(
           [&]() {
             const BatchChains ch = batch_chains(b);
             hipError_t e = fork_chains(b, ch);
-            if (e == hipSuccess)
+            for (int st = 0; st < batch_nstages(b) && e == hipSuccess; ++st)
               e = launch_batch_kernels(b, a, grid_for(d, b->ntasks), ch);
             const hipError_t ej = join_chains(b, ch);
             return e == hipSuccess ? ej : e;

@@ -1,5 +1,6 @@
-"""Mixed batches in the serving loop's default precision (FP32 rates):
-every member takes the bits it takes alone."""
+"""Mixed batches in the serving loop's default precision (FP32 rates) and
+under the autotuner's trials of whole steps: every member takes the bits it
+takes alone."""
 import numpy as np
 import pytest
 
@@ -57,3 +58,33 @@ def test_fp32_rates_step_as_alone(members):
         sub.close()
     dev.close()
 
+
+@pytest.mark.parametrize("prec", [bx.FP32, bx.FP32_RHS, bx.FP64])
+@pytest.mark.parametrize("members", SETS[1:], ids=lambda m: "-".join(str(n) for n, _ in m))
+def test_trials_of_the_strategy_leave_no_trace(members, prec):
+    """Every order on the line kernel, so that the autotuner times the two
+    strategies, in the middle of a step: the run goes on as without it."""
+    print(f"strategy trials {members} prec={prec}", flush=True)
+    dev = bx.Device(0)
+    for N, _ in members:
+        dev.set_kernel(prec, N, 0)
+    cfgs, subs = _members(dev, members, prec)
+    _reset(cfgs, subs)
+    alone = []
+    for sub in subs:
+        sub.step(4)
+        alone.append(sub.download())
+    _reset(cfgs, subs)
+    for sub in subs:
+        for _ in range(7):
+            sub.stage()
+    b = bx.Batch(dev, subs)
+    b.autotune(2)
+    b.step(2)
+    b.close()
+    for sub, q in zip(subs, alone):
+        for _ in range(3):
+            sub.stage()
+        np.testing.assert_array_equal(sub.download(), q)
+        sub.close()
+    dev.close()
