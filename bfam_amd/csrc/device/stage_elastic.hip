@@ -91,16 +91,18 @@ template <int N, int EPB, class P> struct NodeBlock
   static constexpr int value = NodeUnits<N, EPB, P>::value ? (nodes + 63) / 64 * 64 : nodes;
 };
 
-/* Whether a block requests its face indices and D after the state's LDS-DMA
- * and before the barrier.  Otherwise D's round trip through a register comes
- * before the DMA, and the index loads after the barrier, ahead of the
- * gathers.  us per stage, later / here: FP32 N = 3 (30^3) 52.3 / 50.3, N = 5
- * (10^3) 12.65 / 12.41 and (21^3) 58.8 / 58.8, N = 6 (18^3) 72.5 / 63.1, N = 7
- * (32^3) 374 / 371; FP32 rates N = 3 (24^3) 42.1 / 40.4; FP64 N = 5 (18^3)
- * 70.6 / 69.6; but FP32 N = 4 (27^3) 77.0 / 81.4, (46^3) 386 / 410. */
+/* Whether a block with face tasks requests its face indices and D after the
+ * state's LDS-DMA and before the barrier.  Otherwise D's round trip through a
+ * register comes before the DMA, and the index loads after the barrier, ahead
+ * of the gathers.  us per stage, later / here: FP32 N = 3 50.7 / 49.1 (30^3),
+ * N = 6 78.3 / 58.4 (18^3), 381 / 258 (30^3); FP32 rates N = 3 42.1 / 40.2 (24^3),
+ * N = 5 61.0 / 60.3 (18^3), 258 / 258 (30^3); FP64 N = 3 51.6 / 51.1 (24^3), N = 6
+ * 74.5 / 75.4 (16^3); but N = 4 FP32 rates 55.1 / 55.5 (20^3), 223 / 226 (32^3), and
+ * FP32 with four elements a block 90.4 / 93.4 (27^3; FP64 74.9 / 73.9, 20^3) */
 template <int N, class P, bool SPLIT> struct NodeEarly
 {
-  /* the whole-task form of N = 3, at its 80 registers, would spill more */
+  /* the whole-task form of N = 3 (not launched: launch_ne), at its 80
+   * registers, would spill more */
   static constexpr bool value = N != 4 && (N != 3 || SPLIT || !__is_same(P, P32));
 };
 
@@ -851,8 +853,8 @@ template <int N, int EPB, class P> struct NodeWaves
 };
 
 /* elements per block of the fused node-parallel kernel.  A node task holds
- * up to 512 / (N+1)^3 elements (elastic_epb); a block of fewer elements
- * takes a task in passes.  Smaller blocks let more of them share a CU
+ * up to 512 / (N+1)^3 elements (elastic_epb); blocks of fewer elements
+ * share it or take it in passes.  Smaller blocks let more of them share a CU
  * (the LDS of a block scales with its elements), ms per stage on bricks of
  * about 124 M DOF, one-block-per-task grid:
  *   N = 5, one element (216 threads): FP32 0.541 -> 0.483, FP32 rates
@@ -864,7 +866,9 @@ template <int N, int EPB, class P> struct NodeWaves
  *   registers 0.607, at 114 0.610; two elements 0.626).
  * FP32 rates at N = 3, 4 with one element measured slower taking a task
  * in passes (0.708 -> 0.759, 0.894 -> 1.007) and faster with one block per
- * element (NodeSplit): 0.705 -> 0.642, 0.868 -> 0.813. */
+ * element: 0.705 -> 0.642, 0.868 -> 0.813.  Every order below 6 has one block
+ * per EPB elements since (NodeSplit); only the other block size and the
+ * matrix-core derivatives take tasks in passes. */
 template <int N, class P> struct NodeEpb
 {
   static constexpr bool f32 = __is_same(P, P32) || __is_same(P, P32R), f64 = __is_same(P, P64);
@@ -1013,6 +1017,8 @@ static hipError_t launch_ne(const LaunchArgs &a, int grid, hipStream_t s, unsign
                        dim3(NodeBlock<N, EPB, P>::value), dyn, s, a);
     return hipGetLastError();
   }
+  /* NS = 1.  The whole-task form of a split order is compiled, as the one
+   * that its registers are compared with, and never launched */
   hipLaunchKernelGGL((elastic_stage_kernel<N, EPB, P>), dim3(grid),
                      dim3(NodeBlock<N, EPB, P>::value), dyn, s, a);
   return hipGetLastError();
